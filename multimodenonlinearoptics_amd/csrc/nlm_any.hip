@@ -4,6 +4,11 @@
 // kissfft's mixed-radix transform, src/CustomEigenFFT.h:17-40), lengths 2 and
 // 4, and lengths above 8192.
 //
+// Lengths with a plan N = R (small radices) R whose fields and twiddles fit in LDS run
+// the in-register mixed-radix kernels of nlm_mix.hpp (mix_plan below).  The kernels of
+// this file run the others: a large prime factor, no square factor (N = 30), or
+// a field beyond LDS.
+//
 // One workgroup of 256 lanes owns one field at a time (a persistent grid walks
 // the fields).  The field's modes and a second buffer per mode live in LDS when
 // they fit in 64 KB, otherwise in a per-workgroup slice of a device scratch
@@ -22,10 +27,12 @@
 // (solvers/Chi3.cpp:25-54), setPump(other) (src/_NonlinearMedium.cpp:506-534)
 // and the transforms of nlm_fft.
 #include <algorithm>
+#include <cmath>
 #include <cstring>
 #include <string>
 
 #include "nlm_internal.hpp"
+#include "nlm_mix.hpp"
 
 extern __shared__ cplx any_lds[];
 
@@ -426,6 +433,27 @@ int any_plan(int N, AnyFft* f) {
   return NLM_OK;
 }
 
+mix_fn pick_mix(int model, int R) {
+  switch (model) {
+    case NLM_CHI3:
+    case NLM_CHI2PDC: return nlm_pick_mix_1(R);
+    case NLM_CHI2SFG:
+    case NLM_CHI2AFC: return nlm_pick_mix_2(R);
+    case NLM_CHI2SFGPDC: return nlm_pick_mix_4(R);
+    case NLM_CHI2SFGII: return nlm_pick_mix_5(R);
+    case NLM_CHI2PDCII: return nlm_pick_mix_6(R);
+    case NLM_CHI2SFGOPA: return nlm_pick_mix_7(R);
+    case NLM_CHI2SFGXPM: return nlm_pick_mix_8(R);
+    case NLM_CHI2SHG:
+    case NLM_CHI2ASHG: return nlm_pick_mix_9(R);
+    case NLM_CHI2SHGOPA: return nlm_pick_mix_10(R);
+    case NLM_CHI2DSFG: return nlm_pick_mix_11(R);
+    case NLM_CHI2SHGXPM: return nlm_pick_mix_12(R);
+    case NLM_CHI3GNLSE: return nlm_pick_mix_14(R);
+  }
+  return nullptr;
+}
+
 // Launch shape: a persistent grid over `items`, LDS workspaces when 2 NS N
 // points fit in 64 KB, else a device scratch of grid x 2 NS N points held by the
 // plan (or by `own` when there is no plan).
@@ -504,6 +532,26 @@ int nlm_any_prop(nlm_plan_s* p, const KParams& kp, bool may_alloc) {
   const any_prop_fn fn = pick_any_prop(p->model);
   if (!fn) return set_err(NLM_INVALID_ARGUMENT, "unsupported model");
   if (kp.nFields <= 0) return NLM_OK;
+  MixPlan mp;
+  const bool oneMode = p->model == NLM_CHI3 || p->model == NLM_CHI2PDC;
+  // the one-mode media's mixed-radix kernel applies the step table, which needs a
+  // device buffer
+  if ((!oneMode || (p->stepTable && may_alloc)) &&
+      mix_plan(p->N, p->nS, kp.nFields, p->model == NLM_CHI3GNLSE, &mp)) {
+    const mix_fn mf = pick_mix(p->model, mp.R);
+    if (!mf) return set_err(NLM_INVALID_ARGUMENT, "unsupported model / size");
+    if (int e = get_twiddles(p->N, &mp.tw)) return e;
+    KParams kq = kp;
+    if (oneMode) {
+      if (int e = p->stepTab.ensure((size_t)p->nZ * p->N * 2)) return e;
+      nlm_launch_step_table(p->model, p->coef.p, p->cconst.p, p->pumpT[0].p, p->N, p->nZ, p->stepTab.p, p->stream);
+      HIP_TRY(hipGetLastError());
+      kq.tab = p->stepTab.p;
+    }
+    mf(kq, mp, (kp.nFields + mp.FPB - 1) / mp.FPB, p->stream);
+    HIP_TRY(hipGetLastError());
+    return NLM_OK;
+  }
   AnyFft f;
   if (int e = any_plan(p->N, &f)) return e;
   AnyLaunch al;
@@ -518,6 +566,28 @@ int nlm_any_prop(nlm_plan_s* p, const KParams& kp, bool may_alloc) {
 
 int nlm_any_pump_linear(nlm_plan_s* p, const double* strength_dev, double dzp) {
   const int N = p->N, nZP = 2 * p->nZ - 1;
+  MixPlan mp;
+  if (mix_plan(N, 1, nZP, false, &mp)) {
+    if (int e = get_twiddles(N, &mp.tw)) return e;
+    MixRows r{};
+    r.in = p->env.p;
+    r.out = p->F0.p;
+    r.count = p->nP;
+    nlm_mix_rows(MIX_ROWS_FFT, r, mp, p->stream);
+    r.dzp = dzp;
+    r.strength = strength_dev;
+    r.nZP = nZP;
+    for (int q = 0; q < p->nP; q++) {
+      r.F0 = p->F0.p + (size_t)q * N;
+      r.env = p->env.p + (size_t)q * N;
+      r.Dp = p->Dp.p + (size_t)q * N;
+      r.pumpF = p->pumpF[q].p;
+      r.pumpT = p->pumpT[q].p;
+      nlm_mix_rows(MIX_ROWS_LINEAR, r, mp, p->stream);
+    }
+    HIP_TRY(hipGetLastError());
+    return NLM_OK;
+  }
   AnyFft f;
   if (int e = any_plan(N, &f)) return e;
   AnyLaunch al;
@@ -534,6 +604,22 @@ int nlm_any_pump_linear(nlm_plan_s* p, const double* strength_dev, double dzp) {
 
 int nlm_any_pump_chi3(nlm_plan_s* p, double dzp) {
   const int N = p->N, nZP = 2 * p->nZ - 1;
+  MixPlan mp;
+  if (mix_plan(N, 1, 1, false, &mp)) {
+    if (int e = get_twiddles(N, &mp.tw)) return e;
+    MixRows r{};
+    r.env = p->env.p;
+    r.Dp = p->Dp.p;
+    r.dzp = dzp;
+    r.dstepP = p->dsp.p;
+    r.relI = p->relI.p;
+    r.nZP = nZP;
+    r.pumpF = p->pumpF[0].p;
+    r.pumpT = p->pumpT[0].p;
+    nlm_mix_rows(MIX_ROWS_CHI3, r, mp, p->stream);
+    HIP_TRY(hipGetLastError());
+    return NLM_OK;
+  }
   AnyFft f;
   if (int e = any_plan(N, &f)) return e;
   AnyLaunch al;
@@ -558,9 +644,21 @@ int nlm_any_pump_import(nlm_plan_s* p, int q, const cplx* sigF, int nzs, double 
 }
 
 int nlm_any_fft(const cplx* in, cplx* out, int n, int count, bool inverse, hipStream_t s, DevBuf<cplx>* scratch) {
+  if (count <= 0) return NLM_OK;
+  MixPlan mp;
+  if (mix_plan(n, 1, count, false, &mp)) {
+    if (int e = get_twiddles(n, &mp.tw)) return e;
+    MixRows r{};
+    r.in = in;
+    r.out = out;
+    r.count = count;
+    r.inverse = inverse ? 1 : 0;
+    nlm_mix_rows(MIX_ROWS_FFT, r, mp, s);
+    HIP_TRY(hipGetLastError());
+    return NLM_OK;
+  }
   AnyFft f;
   if (int e = any_plan(n, &f)) return e;
-  if (count <= 0) return NLM_OK;
   AnyLaunch al;
   if (int e = any_launch(nullptr, scratch, 1, n, count, &al)) return e;
   hipLaunchKernelGGL(k_any_fft, dim3(al.grid), dim3(ANY_THREADS), al.lds, s, in, out, count, inverse ? 1 : 0, f,
