@@ -82,7 +82,7 @@ def build(force=False, jobs=None, verbose=False):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_compose.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_any.o")
     objs.append(o)
-    deps = _deps("nlm_any.hip", "nlm_mix.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_any.hip", "nlm_mix.hpp", "nlm_modes.hpp", "nlm_internal.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_any.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_noalloc.o")
@@ -107,7 +107,7 @@ def build(force=False, jobs=None, verbose=False):
     for m in PROP_MODELS:
         o = os.path.join(OBJ, "nlm_prop_%d.o" % m)
         objs.append(o)
-        deps = _deps("nlm_prop_inst.hip", *dev_hdrs)
+        deps = _deps("nlm_prop_inst.hip", "nlm_modes.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_INST_MODEL=%d" % m, "-c",
                                                 os.path.join(CSRC, "nlm_prop_inst.hip"), "-o", o])
@@ -120,13 +120,13 @@ def build(force=False, jobs=None, verbose=False):
                                                 os.path.join(CSRC, "nlm_multi_inst.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_mix_rows.o")
     objs.append(o)
-    deps = _deps("nlm_mix_rows.hip", "nlm_mix.hpp", *dev_hdrs)
+    deps = _deps("nlm_mix_rows.hip", "nlm_mix.hpp", "nlm_modes.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_mix_rows.hip"), "-o", o])
     for m in PROP_MODELS[1:]:  # mixed-radix kernels (id 1: the step table of Chi3 and Chi2PDC)
         o = os.path.join(OBJ, "nlm_mix_%d.o" % m)
         objs.append(o)
-        deps = _deps("nlm_mix_inst.hip", "nlm_mix.hpp", *dev_hdrs)
+        deps = _deps("nlm_mix_inst.hip", "nlm_mix.hpp", "nlm_modes.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_INST_MODEL=%d" % m, "-c",
                                                 os.path.join(CSRC, "nlm_mix_inst.hip"), "-o", o])

@@ -226,6 +226,42 @@ struct TableTwiddles {
   }
 };
 
+// For lanes with 128 registers: the first stage's twiddles W_N^(t c) in registers, the
+// later stages' in a compact LDS table, entry (c - 1) M + b of stage s = W_N^(b c P)
+// (504 entries at N = 4096).
+template <int L>
+struct StageTwiddles {
+  using F = FftShape<L>;
+  static constexpr int stage_len(int s) { return F::N / F::before(s) / F::radix(s); }  // M
+  static constexpr int offset(int s) {  // of stage s >= 1
+    int o = 0;
+    for (int i = 1; i < s; i++) o += (F::radix(i) - 1) * stage_len(i);
+    return o;
+  }
+  static constexpr int ELEMS = offset(F::S - 1);  // the last stage has none
+  cplx w0[8];
+  const cplx* tab;
+  int t;
+  __device__ __forceinline__ void init(cplx* lds, const cplx* table, int t_) {
+    t = t_;
+    tab = lds;
+#pragma unroll
+    for (int c = 1; c < 8; c++) w0[c] = table[t_ * c];
+#pragma unroll
+    for (int s = 1; s < F::S - 1; s++) {
+      const int M = stage_len(s), cnt = (F::radix(s) - 1) * M;
+      for (int k = threadIdx.x; k < cnt; k += blockDim.x)
+        lds[offset(s) + k] = table[(k % M) * (k / M + 1) * F::before(s)];
+    }
+  }
+  __device__ __forceinline__ cplx operator()(int s, int idx) const {
+    if (s == 0) return w0[idx];
+    const int R = F::radix(s), M = stage_len(s);
+    const int j = idx / R, c = idx % R;
+    return tab[offset(s) + (c - 1) * M + (t + F::T * j) % M];
+  }
+};
+
 // Twiddles of the propagation kernels.  Up to N = 2048 a field's lanes have 512
 // registers each (one wave per SIMD) and keep their twiddles in registers.  From
 // N = 4096 a field needs 512 or 1024 lanes, i.e. two or four waves per SIMD with
@@ -410,12 +446,20 @@ __device__ __forceinline__ void fft_field2(cplx (&v)[8], cplx (&u)[8], cplx* __r
   }
 }
 
-// One field with twiddles from tw(s, idx) (see fft_field).
-template <int L, bool INV, int s, bool WAVE = false, class TW>
-__device__ __forceinline__ void fft_stages1(cplx (&v)[8], cplx* __restrict__ buf, int t, const TW& tw) {
+struct NoFetch {
+  __device__ __forceinline__ void operator()() const {}
+};
+
+// One field with twiddles from tw(s, idx) (see fft_field).  `fetch` runs before the
+// last exchange's reads: loads issued there are covered by the last stage, and their
+// registers are not live through the earlier ones.
+template <int L, bool INV, int s, bool WAVE = false, class TW, class Fetch = NoFetch>
+__device__ __forceinline__ void fft_stages1(cplx (&v)[8], cplx* __restrict__ buf, int t, const TW& tw,
+                                            const Fetch& fetch = Fetch()) {
   using F = FftShape<L>;
   constexpr int N = F::N, T = F::T, S = F::S;
   constexpr int R = F::radix(s), P = F::before(s), Mp = N / P, M = Mp / R, NB = 8 / R;
+  if constexpr (s == S - 1) fetch();
   exchange_sync<WAVE>();
 #pragma unroll
   for (int j = 0; j < NB; j++) {
@@ -446,21 +490,23 @@ __device__ __forceinline__ void fft_stages1(cplx (&v)[8], cplx* __restrict__ buf
       for (int c = 0; c < R; c++)
         buf[lpad<L>((g + P * c) * M + b)] = c == 0 ? v[j * R] : twmul<INV>(v[j * R + c], tw(s, j * R + c));
     }
-    fft_stages1<L, INV, s + 1, WAVE>(v, buf, t, tw);
+    fft_stages1<L, INV, s + 1, WAVE>(v, buf, t, tw, fetch);
   }
 }
 
-template <int L, bool INV, bool WAVE = false, class TW>
-__device__ __forceinline__ void fft_field1(cplx (&v)[8], cplx* __restrict__ buf, int t, const TW& tw) {
+template <int L, bool INV, bool WAVE = false, class TW, class Fetch = NoFetch>
+__device__ __forceinline__ void fft_field1(cplx (&v)[8], cplx* __restrict__ buf, int t, const TW& tw,
+                                           const Fetch& fetch = Fetch()) {
   using F = FftShape<L>;
   constexpr int T = F::T, S = F::S;
   dft_small<8, INV>(v);
+  if constexpr (S == 1) fetch();
   if constexpr (S > 1) {
 #pragma unroll
     for (int c = 1; c < 8; c++) v[c] = twmul<INV>(v[c], tw(0, c));
     exchange_sync<WAVE>();
 #pragma unroll
     for (int c = 0; c < 8; c++) buf[lpad<L>(c * T + t)] = v[c];
-    fft_stages1<L, INV, 1, WAVE>(v, buf, t, tw);
+    fft_stages1<L, INV, 1, WAVE>(v, buf, t, tw, fetch);
   }
 }

@@ -12,9 +12,7 @@
 // round trip per stage boundary.  R is a template parameter (register arrays), the
 // middle radices and N are kernel arguments.
 //
-// Every signal mode of a medium has lanes of its own (a group), so the modes'
-// transforms run side by side; for the RK4 step the groups exchange the modes'
-// points through LDS and each group evaluates a share of the points.
+// Every signal mode of a medium has lanes of its own (nlm_modes.hpp).
 //
 // What bounds it: like every kernel of this engine, a wave's FP64 instructions (4
 // cycles each) plus its 16-byte LDS accesses (~30 cycles each when nothing else runs
@@ -31,7 +29,7 @@
 #include <algorithm>
 #include <cmath>
 
-#include "nlm_prop.hpp"
+#include "nlm_modes.hpp"
 
 constexpr int MIX_MAX_MID = 3;
 constexpr int MIX_MAX_THREADS = 512;  // two waves per SIMD: 256 registers per lane
@@ -131,10 +129,7 @@ extern __shared__ cplx mix_lds[];
 
 namespace mix {
 
-__device__ __forceinline__ void sync_if(bool wave) {
-  if (wave) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
-  else lds_barrier();
-}
+using namespace modes;
 
 // R-point DFT in place, natural order in and out; forward exp(-2 pi i nk/R).
 template <int R, bool INV>
@@ -248,8 +243,9 @@ __device__ __forceinline__ void dft(cplx* v) {
 
 // One group's view of its field: lane j of the T that hold a mode, its LDS buffer
 // and the first stage's twiddles W_N^(j c).
-template <int R>
+template <int RADIX>
 struct Fft {
+  static constexpr int R = RADIX;
   const MixPlan& p;
   cplx* buf;
   const cplx* tab;  // LDS copy of W_N^m
@@ -268,7 +264,11 @@ struct Fft {
   }
 
   __device__ __forceinline__ int at(int k) const { return j + p.T * k; }
+  __device__ __forceinline__ int n() const { return p.N; }
+  __device__ __forceinline__ double invN() const { return p.invN; }
+  __device__ __forceinline__ int bufElems() const { return p.bufElems; }
   __device__ __forceinline__ void sync() const { sync_if(p.waveFft); }
+  __device__ __forceinline__ void syncAll() const { sync_if(p.waveAll); }
 
   // Middle stage of radix Q: butterflies beta = j, j + TP, ... read [g][a][b]
   // (sub-arrays g of Q M points), write [g + P c][b]; `pitch` is the written
@@ -406,91 +406,6 @@ __device__ __forceinline__ const cplx* load_table(const MixPlan& p, cplx* lds) {
   return lds;
 }
 
-template <int R>
-__device__ __forceinline__ void put_row(const Fft<R>& f, cplx* __restrict__ dst, const cplx (&v)[R], bool act) {
-  if (act)
-#pragma unroll
-    for (int k = 0; k < R; k++) dst[f.at(k)] = v[k];
-}
-template <int R>
-__device__ __forceinline__ void put_scaled(const Fft<R>& f, cplx* __restrict__ dst, const cplx (&v)[R], bool act) {
-  const double s = f.p.invN;
-  if (act)
-#pragma unroll
-    for (int k = 0; k < R; k++) dst[f.at(k)] = v[k] * s;
-}
-template <int R>
-__device__ __forceinline__ void get_row(const Fft<R>& f, cplx (&v)[R], const cplx* __restrict__ src) {
-#pragma unroll
-  for (int k = 0; k < R; k++) v[k] = src[f.on ? f.at(k) : 0];
-}
-template <int R>
-__device__ __forceinline__ void mul_row(const Fft<R>& f, cplx (&v)[R], const cplx* __restrict__ tab) {
-#pragma unroll
-  for (int k = 0; k < R; k++) v[k] = v[k] * tab[f.on ? f.at(k) : 0];
-}
-template <int R>
-__device__ __forceinline__ void scale_row(const Fft<R>& f, cplx (&v)[R]) {
-#pragma unroll
-  for (int k = 0; k < R; k++) v[k] = v[k] * f.p.invN;
-}
-
-template <int NS>
-__device__ __forceinline__ int of_mode(const int (&a)[4], int g) {
-  int r = a[0];
-#pragma unroll
-  for (int q = 1; q < NS; q++) r = g == q ? a[q] : r;
-  return r;
-}
-
-// Input of mode g and the half dispersion step in (src/_NonlinearMedium.hpp:164-198,
-// src/_NonlinearMedium.cpp:329-340); leaves the spectrum.
-template <int NS, int R>
-__device__ __forceinline__ void enter(const KParams& kp, Fft<R>& f, int field, int g, bool act, cplx (&v)[R]) {
-  const int N = f.p.N;
-#pragma unroll
-  for (int k = 0; k < R; k++) v[k] = mk(0.0, 0.0);
-  if (act) {
-    if (kp.kind == KIND_GREENS) {
-      const int i = field >> 1, w = field & 1, src = i / N, pos = i - src * N;
-      const cplx val = w ? mk(0.0, 1.0) : mk(1.0, 0.0);
-      if (kp.inputs[src] == g)
-#pragma unroll
-        for (int k = 0; k < R; k++)
-          if (f.at(k) == pos) v[k] = val;
-    } else {
-      const int ch = of_mode<NS>(kp.inPos, g);
-      if (ch >= 0) {
-        const cplx* row = kp.in + (size_t)field * kp.inCols + (size_t)ch * N;
-#pragma unroll
-        for (int k = 0; k < R; k++) v[k] = row[f.at(k)];
-      }
-    }
-  }
-  if (kp.inTime) f.template run<false>(v);
-  mul_row<R>(f, v, kp.halfIn + (size_t)g * N);
-  if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridF, field, NS, g, 0, N), v, act);
-}
-
-// Half step out and outputs (src/_NonlinearMedium.hpp:235-238, src/_NonlinearMedium.cpp:333-345, 428-431).
-template <int NS, int R>
-__device__ __forceinline__ void leave(const KParams& kp, Fft<R>& f, int field, int g, bool act, cplx (&v)[R]) {
-  const int N = f.p.N, last = kp.nZ - 1;
-  mul_row<R>(f, v, kp.halfOut + (size_t)g * N);
-  if (kp.kind == KIND_GRID) {
-    put_row<R>(f, grid_row(kp, kp.gridF, field, NS, g, last, N), v, act);
-    f.template run<true>(v);
-    put_scaled<R>(f, grid_row(kp, kp.gridT, field, NS, g, last, N), v, act);
-  } else {
-    if (kp.outTime) {
-      f.template run<true>(v);
-      scale_row<R>(f, v);
-    }
-    const int op = of_mode<NS>(kp.outPos, g);
-    if (op >= 0) put_row<R>(f, kp.out + (size_t)field * kp.nOut * N + (size_t)op * N, v, act);
-  }
-}
-
 // A one-mode medium whose RK4 step is the real 2x2 matrix of kp.tab (see
 // nlm_prop_tab.hip; the table holds the inverse transform's 1/N).
 struct Table {
@@ -512,11 +427,11 @@ template <int R>
 __device__ __forceinline__ void table_field(const KParams& kp, Fft<R>& f, int field, bool act) {
   const int N = f.p.N;
   cplx v[R];
-  enter<1, R>(kp, f, field, 0, act, v);
+  enter<1>(kp, f, field, 0, act, v);
   cplx al[R], be[R];
   if (kp.nZ > 1) {
     f.template run<true>(v);
-    if (kp.kind == KIND_GRID) put_scaled<R>(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), v, act);
+    if (kp.kind == KIND_GRID) put_scaled(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), v, act);
     get_matrices<R>(f, al, be, kp.tab + (size_t)N * 2);
   }
   for (int i = 1; i < kp.nZ; i++) {
@@ -526,121 +441,14 @@ __device__ __forceinline__ void table_field(const KParams& kp, Fft<R>& f, int fi
       v[k] = mk(al[k].re * x.re + al[k].im * x.im, be[k].re * x.re + be[k].im * x.im);
     }
     f.template run<false>(v);
-    mul_row<R>(f, v, kp.dstep);
+    mul_row(f, v, kp.dstep);
     if (i < kp.nZ - 1) {
-      if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
-      f.template run<true>(v, [&] { get_matrices<R>(f, al, be, kp.tab + (size_t)(i + 1) * N * 2); });
-      if (kp.kind == KIND_GRID) put_scaled<R>(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), v, act);
+      if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
+      f.template run<true>(v, [&]() __attribute__((always_inline)) { get_matrices<R>(f, al, be, kp.tab + (size_t)(i + 1) * N * 2); });
+      if (kp.kind == KIND_GRID) put_scaled(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), v, act);
     }
   }
-  leave<1, R>(kp, f, field, 0, act, v);
-}
-
-// One mode (group g) of a propagation of a pointwise model with NS >= 2 modes.
-template <class M, int R>
-__device__ __forceinline__ void modes_field(const KParams& kp, Fft<R>& f, cplx* fieldBuf, int field, int g, bool act) {
-  constexpr int NS = M::NS, NP = M::NP, NC = M::NC, NPP = NP > 0 ? NP : 1;
-  constexpr int KS = (R + NS - 1) / NS;  // points of this group's share: k = kk NS + g
-  const int N = f.p.N;
-  cplx v[R];
-  enter<NS, R>(kp, f, field, g, act, v);
-  if (kp.nZ > 1) {
-    f.template run<true>(v);
-    scale_row<R>(f, v);
-    if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridT, field, NS, g, 0, N), v, act);
-  }
-  // the share's pump rows 2i-2 (pp), 2i-1 (pi), 2i (pc) of step i
-  cplx pp[NPP][KS], pi[NPP][KS], pc[NPP][KS];
-  const cplx* pumps[2] = {kp.pump0, kp.pump1};
-  auto pump = [&](cplx (&dst)[KS], const cplx* row) {
-#pragma unroll
-    for (int kk = 0; kk < KS; kk++) {
-      const int k = kk * NS + g;
-      dst[kk] = row[f.on && k < R ? f.at(k) : 0];
-    }
-  };
-#pragma unroll
-  for (int r = 0; r < NP; r++) {
-    pump(pp[r], pumps[r]);
-    if (kp.nZ > 1) {
-      pump(pi[r], pumps[r] + N);
-      pump(pc[r], pumps[r] + (size_t)2 * N);
-    }
-  }
-  constexpr int NCC = M::NCC > 0 ? M::NCC : 1;
-  cplx cc[NCC];
-  {
-    const uniform_cplx* ccq = to_uniform(kp.cconst);
-#pragma unroll
-    for (int k = 0; k < M::NCC; k++) cc[k] = mk(ccq[k].re, ccq[k].im);
-  }
-  for (int i = 1; i < kp.nZ; i++) {
-    // --- RK4 step: every group offers its mode's points, takes all modes of its
-    // share, and returns them
-    f.sync();  // the transform's readers of this group's buffer are done
-    if (f.on)
-#pragma unroll
-      for (int k = 0; k < R; k++) f.buf[f.at(k)] = v[k];
-    sync_if(f.p.waveAll);
-    cplx c[3 * NC];
-    {
-      const uniform_cplx* cq = to_uniform(kp.coef + (size_t)i * 3 * NC);
-#pragma unroll
-      for (int k = 0; k < 3 * NC; k++) c[k] = mk(cq[k].re, cq[k].im);
-    }
-#pragma unroll
-    for (int kk = 0; kk < KS; kk++) {
-      const int k = kk * NS + g;
-      if (f.on && k < R) {
-        const int at = f.at(k);
-        cplx x[NS], y[NS], k1[NS], k2[NS], k3[NS], k4[NS], P0[NPP], P1[NPP], P2[NPP];
-#pragma unroll
-        for (int r = 0; r < NPP; r++) {
-          P0[r] = NP ? pp[r][kk] : mk(0, 0);
-          P1[r] = NP ? pi[r][kk] : mk(0, 0);
-          P2[r] = NP ? pc[r][kk] : mk(0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q < NS; q++) x[q] = fieldBuf[q * f.p.bufElems + at];
-        M::template f<0>(c, cc, x, P0, k1);
-#pragma unroll
-        for (int q = 0; q < NS; q++) y[q] = x[q] + 0.5 * k1[q];
-        M::template f<1>(c + NC, cc, y, P1, k2);
-#pragma unroll
-        for (int q = 0; q < NS; q++) y[q] = x[q] + 0.5 * k2[q];
-        M::template f<2>(c + NC, cc, y, P1, k3);
-#pragma unroll
-        for (int q = 0; q < NS; q++) y[q] = x[q] + k3[q];
-        M::template f<3>(c + 2 * NC, cc, y, P2, k4);
-#pragma unroll
-        for (int q = 0; q < NS; q++)
-          fieldBuf[q * f.p.bufElems + at] =
-              x[q] + (((k1[q] + 2.0 * k2[q]) + 2.0 * k3[q]) + k4[q]) * (1. / 6.);
-      }
-    }
-    sync_if(f.p.waveAll);
-    if (f.on)
-#pragma unroll
-      for (int k = 0; k < R; k++) v[k] = f.buf[f.at(k)];
-    // --- dispersion step (src/_NonlinearMedium.hpp:212-215)
-    f.template run<false>(v);
-    mul_row<R>(f, v, kp.dstep + (size_t)g * N);
-    if (i < kp.nZ - 1) {
-      if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridF, field, NS, g, i, N), v, act);
-      f.template run<true>(v, [&] {
-#pragma unroll
-        for (int r = 0; r < NP; r++) {
-#pragma unroll
-          for (int kk = 0; kk < KS; kk++) pp[r][kk] = pc[r][kk];
-          pump(pi[r], pumps[r] + (size_t)(2 * i + 1) * N);
-          pump(pc[r], pumps[r] + (size_t)(2 * i + 2) * N);
-        }
-      });
-      scale_row<R>(f, v);
-      if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridT, field, NS, g, i, N), v, act);
-    }
-  }
-  leave<NS, R>(kp, f, field, g, act, v);
+  leave<1>(kp, f, field, 0, act, v);
 }
 
 // k = IFFT( FFT( IFFT(FFT(r |y|^2) * R) * y ) * (nl0 + nl1*omega) ), solvers/Chi3GNLSE.cpp:51-92
@@ -649,26 +457,26 @@ __device__ __forceinline__ void gnlse_stage(const KParams& kp, Fft<R>& f, const 
 #pragma unroll
   for (int m = 0; m < R; m++) k[m] = mk(r * abs2(y[m]), 0.0);
   f.template run<false>(k);
-  mul_row<R>(f, k, kp.raman);
+  mul_row(f, k, kp.raman);
   f.template run<true>(k);
-  scale_row<R>(f, k);
+  scale_row(f, k);
 #pragma unroll
   for (int m = 0; m < R; m++) k[m] = k[m] * y[m];
   f.template run<false>(k);
-  mul_row<R>(f, k, kp.filt);
+  mul_row(f, k, kp.filt);
   f.template run<true>(k);
-  scale_row<R>(f, k);
+  scale_row(f, k);
 }
 
 template <int R>
 __device__ __forceinline__ void gnlse_field(const KParams& kp, Fft<R>& f, int field, bool act) {
   const int N = f.p.N;
   cplx v[R];
-  enter<1, R>(kp, f, field, 0, act, v);
+  enter<1>(kp, f, field, 0, act, v);
   if (kp.nZ > 1) {
     f.template run<true>(v);
-    scale_row<R>(f, v);
-    if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), v, act);
+    scale_row(f, v);
+    if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), v, act);
   }
   for (int i = 1; i < kp.nZ; i++) {
     const uniform_cplx* c = to_uniform(kp.coef + (size_t)i * 3);
@@ -694,15 +502,15 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, Fft<R>& f, int fi
 #pragma unroll
     for (int m = 0; m < R; m++) v[m] = v[m] + acc[m] * (1. / 6.);
     f.template run<false>(v);
-    mul_row<R>(f, v, kp.dstep);
+    mul_row(f, v, kp.dstep);
     if (i < kp.nZ - 1) {
-      if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
+      if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
       f.template run<true>(v);
-      scale_row<R>(f, v);
-      if (kp.kind == KIND_GRID) put_row<R>(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), v, act);
+      scale_row(f, v);
+      if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), v, act);
     }
   }
-  leave<1, R>(kp, f, field, 0, act, v);
+  leave<1>(kp, f, field, 0, act, v);
 }
 
 }  // namespace mix
@@ -718,7 +526,7 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_prop(KParams kp, MixPla
   const bool act = f.on && field < kp.nFields;
   if constexpr (std::is_same<M, mix::Table>::value) mix::table_field<R>(kp, f, field, act);
   else if constexpr (std::is_same<M, MChi3GNLSE>::value) mix::gnlse_field<R>(kp, f, field, act);
-  else mix::modes_field<M, R>(kp, f, fieldBuf, field, a.g, act);
+  else modes::modes_field<M>(kp, f, fieldBuf, field, a.g, act);
 }
 
 typedef void (*mix_fn)(const KParams&, const MixPlan&, int grid, hipStream_t);

@@ -11,13 +11,13 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_fft(MixRows r, MixPlan 
   const int row = blockIdx.x * p.FPB + a.slot;
   const bool act = f.on && row < r.count;
   cplx v[R];
-  mix::get_row<R>(f, v, r.in + (size_t)(act ? row : 0) * p.N);
+  mix::get_row(f, v, r.in + (size_t)(act ? row : 0) * p.N);
   if (r.inverse) {
     f.template run<true>(v);
-    mix::put_scaled<R>(f, r.out + (size_t)row * p.N, v, act);
+    mix::put_scaled(f, r.out + (size_t)row * p.N, v, act);
   } else {
     f.template run<false>(v);
-    mix::put_row<R>(f, r.out + (size_t)row * p.N, v, act);
+    mix::put_row(f, r.out + (size_t)row * p.N, v, act);
   }
 }
 
@@ -53,8 +53,8 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_pump_linear(MixRows r, 
       t[k] = t[k] * s;
     }
   }
-  mix::put_row<R>(f, r.pumpF + (size_t)i * p.N, v, act);
-  mix::put_row<R>(f, r.pumpT + (size_t)i * p.N, t, act);
+  mix::put_row(f, r.pumpF + (size_t)i * p.N, v, act);
+  mix::put_row(f, r.pumpT + (size_t)i * p.N, t, act);
 }
 
 // The nonlinear pump, serial over its 2nZ-1 rows in one workgroup.
@@ -65,8 +65,8 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_pump_chi3(MixRows r, Mi
   mix::Fft<R> f(p, mix_lds + p.N + (size_t)a.slot * p.bufElems, tab, a.j);
   const bool act = f.on && a.slot == 0;
   cplx v[R], dsp[R];
-  mix::get_row<R>(f, v, r.env);
-  mix::get_row<R>(f, dsp, r.dstepP);
+  mix::get_row(f, v, r.env);
+  mix::get_row(f, dsp, r.dstepP);
   f.template run<false>(v);
 #pragma unroll
   for (int k = 0; k < R; k++) {
@@ -74,10 +74,10 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_pump_chi3(MixRows r, Mi
     sincos((0.5 * r.dzp) * r.Dp[f.on ? f.at(k) : 0], &s, &c);
     v[k] = v[k] * mk(c, s);
   }
-  mix::put_row<R>(f, r.pumpF, v, act);
+  mix::put_row(f, r.pumpF, v, act);
   f.template run<true>(v);
-  mix::scale_row<R>(f, v);
-  mix::put_row<R>(f, r.pumpT, v, act);
+  mix::scale_row(f, v);
+  mix::put_row(f, r.pumpT, v, act);
   for (int i = 1; i < r.nZP; i++) {
     const cplx q = r.relI[i - 1];
 #pragma unroll
@@ -99,10 +99,10 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_pump_chi3(MixRows r, Mi
         v[k] = v[k] * mk(c, s);
       }
     }
-    mix::put_row<R>(f, r.pumpF + (size_t)i * p.N, v, act);
+    mix::put_row(f, r.pumpF + (size_t)i * p.N, v, act);
     f.template run<true>(v);
-    mix::scale_row<R>(f, v);
-    mix::put_row<R>(f, r.pumpT + (size_t)i * p.N, v, act);
+    mix::scale_row(f, v);
+    mix::put_row(f, r.pumpT + (size_t)i * p.N, v, act);
   }
 }
 

@@ -1,6 +1,6 @@
 // nlm_prop_inst.hip -- instantiates the propagation kernel of one model for
 // every supported size.  Compiled once per model with -DNLM_INST_MODEL=<id>.
-#include "nlm_prop.hpp"
+#include "nlm_modes.hpp"
 
 #ifndef NLM_INST_MODEL
 #error "NLM_INST_MODEL must be defined"
@@ -9,7 +9,14 @@
 template <int MODEL, int L>
 static prop_fn pick_L() {
   if constexpr (MODEL == NLM_CHI3GNLSE) return &launch_gnlse<L>;
-  else return &launch_prop<typename ModelOf<MODEL>::type, L>;
+  else {
+    using M = typename ModelOf<MODEL>::type;
+    if constexpr (M::NS > 1)
+      if constexpr (modes::Pow2<L, M::NS>::OK) {
+        return &modes::launch_prop_modes<M, L>;
+      }
+    return &launch_prop<M, L>;
+  }
 }
 
 #define NLM_CAT2(a, b) a##b
