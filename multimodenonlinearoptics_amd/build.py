@@ -93,14 +93,14 @@ def build(force=False, jobs=None, verbose=False):
     for v in range(4):  # FFT schedule variants of the step-table kernel (chosen by the autotuner)
         o = os.path.join(OBJ, "nlm_prop_tab_v%d.o" % v)
         objs.append(o)
-        deps = _deps("nlm_prop_tab.hip", *dev_hdrs)
+        deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_TAB_VARIANT=%d" % v, "-c",
                                                 os.path.join(CSRC, "nlm_prop_tab.hip"), "-o", o])
     # the single-wave sizes of the step-table kernel, with the memory-clause scheduler
     o = os.path.join(OBJ, "nlm_prop_tab_small.o")
     objs.append(o)
-    deps = _deps("nlm_prop_tab.hip", *dev_hdrs)
+    deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause", "-DNLM_TAB_SMALL",
                                             "-c", os.path.join(CSRC, "nlm_prop_tab.hip"), "-o", o])

@@ -16,21 +16,7 @@
 // Green's impulses or batch rows.  The propagator also absorbs the inverse
 // transform's 1/N (an exact power of two), so the field between steps is kept
 // unscaled.
-#include "nlm_prop.hpp"
-
-template <class M>
-__device__ __forceinline__ cplx rk4_step(const cplx* c, const cplx* cc, cplx x, cplx P0, cplx P1, cplx P2) {
-  constexpr int NC = M::NC;
-  cplx xs[1] = {x}, y[1], k1[1], k2[1], k3[1], k4[1], p0[1] = {P0}, p1[1] = {P1}, p2[1] = {P2};
-  M::template f<0>(c, cc, xs, p0, k1);
-  y[0] = x + 0.5 * k1[0];
-  M::template f<1>(c + NC, cc, y, p1, k2);
-  y[0] = x + 0.5 * k2[0];
-  M::template f<2>(c + NC, cc, y, p1, k3);
-  y[0] = x + k3[0];
-  M::template f<3>(c + 2 * NC, cc, y, p2, k4);
-  return x + (((k1[0] + 2.0 * k2[0]) + 2.0 * k3[0]) + k4[0]) * (1. / 6.);
-}
+#include "nlm_tab.hpp"
 
 // tab[(i*N + k)*2 + {0,1}] = {(Re R(1), Re R(i)), (Im R(1), Im R(i))} * scale for
 // steps i = 1..nZ-1: Re x' = p.re Re x + p.im Im x, Im x' = q.re Re x + q.im Im x.
@@ -52,105 +38,40 @@ __global__ void k_step_table(const cplx* __restrict__ coef, const cplx* __restri
   tab[((size_t)i * N + k) * 2 + 1] = mk(scale * r1.im, scale * ri.im);
 }
 
-template <int L>
-__device__ __forceinline__ void load_prop_row(cplx (&al)[8], cplx (&be)[8], const cplx* __restrict__ row, int t) {
-  constexpr int T = FftShape<L>::T;
-#pragma unroll
-  for (int m = 0; m < 8; m++) {
-    al[m] = row[(size_t)(t + T * m) * 2];
-    be[m] = row[(size_t)(t + T * m) * 2 + 1];
-  }
-}
-
-template <int L>
-__device__ __forceinline__ void store_scaled(cplx* __restrict__ dst, const cplx (&v)[8], int t, bool active) {
-  constexpr int T = FftShape<L>::T;
-  constexpr double s = 1.0 / FftShape<L>::N;
-  if (active) {
-#pragma unroll
-    for (int m = 0; m < 8; m++) dst[t + T * m] = v[m] * s;
-  }
-}
-
-// Same contract as k_prop (Green's, batch and grid kinds, checkpoints) for a
-// medium with one signal mode and a step propagator table kp.tab.
-template <int L>
-__global__ void __launch_bounds__(Launch<L>::THREADS) k_prop_tab(KParams kp) {
+// WAVES: waves per SIMD asked of the compiler (0: none asked).
+template <int L, bool MANY, int WAVES>
+__global__ void __launch_bounds__((Launch<L>::THREADS), (WAVES)) k_prop_tab(KParams kp) {
   using F = FftShape<L>;
-  constexpr int N = F::N, T = F::T, FPB = Launch<L>::FPB;
+  constexpr int T = F::T, FPB = Launch<L>::FPB;
   __shared__ cplx lds[FPB * F::lds_elems];
-  __shared__ cplx twl[PropTw<L>::LDS_ELEMS];
-  fill_twiddle_lds<L>(twl, kp.tw);
-
+  __shared__ cplx twl[TabPolicy<L, MANY>::TW_ELEMS];
+  if constexpr (TabPolicy<L, MANY>::TW_LDS) fill_twiddle_lds<L>(twl, kp.tw);
   const int lf = threadIdx.x / T, t = threadIdx.x % T;
   const int field = blockIdx.x * FPB + lf;
-  const bool active = field < kp.nFields;
-  cplx* buf = lds + lf * F::lds_elems;
-
-  typename PropTw<L>::type tw;
-  init_twiddles<L>(tw, kp.tw, twl, t);
-  // Where the dispersion row and the next step's propagator rows live (measured
-  // per size on Green's launches).  N = 512 (one wave per field and SIMD): the
-  // dispersion row is read from L1/L2 where it is used and the propagator rows are
-  // fetched after the forward transform, so neither is held in registers across a
-  // whole step; held across the step they spilled to AGPRs (92 register moves per
-  // step, 3 % of the step time).  N = 1024: the late fetch alone is 7 % faster,
-  // the dispersion row read at use too is slower.  N = 2048 is fastest with both
-  // held; from N = 4096 the dispersion row is read at use (PropTw::LEAN).
-  constexpr int LOG = FftShape<L>::LOG;
-  constexpr bool LATE = LOG == 9 || LOG == 10;
-  constexpr bool DS_MEM = LOG == 9 || PropTw<L>::LEAN;
-  cplx ds[DS_MEM ? 1 : 8];
-  if constexpr (!DS_MEM) {
-#pragma unroll
-    for (int m = 0; m < 8; m++) ds[m] = kp.dstep[t + T * m];
-  }
-
-  cplx a[1][8];
-  load_inputs<L, 1>(a, kp, field, t, active);
-  prologue<L, 1>(a, kp, buf, t, tw, field, active);
-  cplx al[8], be[8];
-  if (kp.nZ > 1) {
-    fft_field1<L, true, kWaveFft<L>>(a[0], buf, t, tw);  // unscaled: the table holds the 1/N
-    if (kp.kind == KIND_GRID) store_scaled<L>(grid_row(kp, kp.gridT, field, 1, 0, 0, N), a[0], t, active);
-    if (kp.ckpt) store_scaled<L>(kp.ckpt + (size_t)field * kp.nSeg * N, a[0], t, active);
-    load_prop_row<L>(al, be, kp.tab + (size_t)N * 2, t);
-  }
-
-#ifdef NLM_TAB_SMALL
-  // two steps per iteration let the scheduler overlap one step's last exchange
-  // and stores with the next step's first loads (N = 512: 1.88 against 1.97 ms per
-  // launch, same box; four steps 2.01 ms; from N = 1024 no change)
-#pragma unroll 2
-#endif
-  for (int i = 1; i < kp.nZ; i++) {
-    // --- RK4 nonlinear step as its R-linear propagator (a real 2 x 2 matrix)
-#pragma unroll
-    for (int m = 0; m < 8; m++) {
-      const cplx x = a[0][m];
-      a[0][m] = mk(al[m].re * x.re + al[m].im * x.im, be[m].re * x.re + be[m].im * x.im);
-    }
-    if (!LATE && i + 1 < kp.nZ) load_prop_row<L>(al, be, kp.tab + (size_t)(i + 1) * N * 2, t);
-
-    // --- dispersion step (src/_NonlinearMedium.hpp:212-215)
-    fft_field1<L, false, kWaveFft<L>>(a[0], buf, t, tw);
-#pragma unroll
-    for (int m = 0; m < 8; m++) a[0][m] = a[0][m] * (DS_MEM ? kp.dstep[t + T * m] : ds[DS_MEM ? 0 : m]);
-    if (LATE && i + 1 < kp.nZ) load_prop_row<L>(al, be, kp.tab + (size_t)(i + 1) * N * 2, t);
-    if (i < kp.nZ - 1) {
-      if (kp.kind == KIND_GRID) store_row<L>(grid_row(kp, kp.gridF, field, 1, 0, i, N), a[0], t, active);
-      fft_field1<L, true, kWaveFft<L>>(a[0], buf, t, tw);
-      if (kp.kind == KIND_GRID) store_scaled<L>(grid_row(kp, kp.gridT, field, 1, 0, i, N), a[0], t, active);
-      if (kp.ckpt && i % kp.ckptEvery == 0)
-        store_scaled<L>(kp.ckpt + ((size_t)field * kp.nSeg + i / kp.ckptEvery) * N, a[0], t, active);
-    }
-  }
-  epilogue<L, 1>(a, kp, buf, t, tw, field, active);
+  tab_field<L, MANY>(kp, field, field < kp.nFields, t, lds + lf * F::lds_elems, twl);
 }
 
+template <int L, bool MANY, int WAVES>
+static void launch_tab(const KParams& kp, int grid, hipStream_t s) {
+  hipLaunchKernelGGL((k_prop_tab<L, MANY, WAVES>), dim3(grid), dim3(Launch<L>::THREADS), 0, s, kp);
+}
+
+// The form of a launch (TabPolicy): the two-waves form where it exists and the
+// launch's waves exceed one per SIMD.  N = 1024 with at most one field per CU is
+// scheduled for one wave per SIMD (one field 0.490 -> 0.472 ms of 199 steps, 200
+// fields 0.510 -> 0.493; no gain with 512 fields).
 template <int L>
 static void launch_prop_tab(const KParams& kp, int grid, hipStream_t s) {
-  hipLaunchKernelGGL((k_prop_tab<L>), dim3(grid), dim3(Launch<L>::THREADS), 0, s, kp);
+  constexpr int CUS = 256, SIMDS = 4 * CUS, LOG = FftShape<L>::LOG;
+  if constexpr (TabPolicy<L, false>::HOOK) {
+    launch_tab<L, false, 2>(kp, grid, s);
+  } else if constexpr (TabPolicy<L, true>::HOOK) {
+    if ((long)grid * (Launch<L>::THREADS / 64) > SIMDS) launch_tab<L, true, 2>(kp, grid, s);
+    else if (LOG == 10 && grid <= CUS) launch_tab<L, false, LOG == 10 ? 1 : 0>(kp, grid, s);
+    else launch_tab<L, false, 0>(kp, grid, s);
+  } else {
+    launch_tab<L, false, 0>(kp, grid, s);
+  }
 }
 
 // This file is compiled once per schedule variant NLM_TAB_VARIANT (see FftShape);
