@@ -183,7 +183,7 @@ int nlm_batch_dev(nlm_plan* plan, const double* inputs_dev, int rows, int cols, 
  * run as one captured graph of per-(model, nFreqs) persistent kernels fed by
  * device work queues.  Every solver; nFreqs a power of two, 32..4096.  With
  * `envelope` set, the pump rows of a single linear pump are generated in the
- * kernel from the envelope (src/_NonlinearMedium.cpp:225-250); with it NULL a
+ * launch from the envelope (src/_NonlinearMedium.cpp:225-250); with it NULL a
  * pumped medium's device pump grids are read (they must have been computed:
  * Chi3's nonlinear pump, Chi2SFGOPA's two pumps, or any grid set before).  The
  * plans must outlive the batch.  (Extension: no counterpart in the reference,
@@ -203,10 +203,12 @@ typedef struct {
 } nlm_multi_item;
 typedef struct nlm_multi_s nlm_multi;
 /* autotune (flags): bit 0 time each class alone for a few persistent grid sizes
- * and keep the fastest (once per process and class shape); bit 1 stage the
- * pump rows of nFreqs 4096 classes with a generated pump: each launch first
- * writes their time-domain rows to a device buffer (a quarter of the device
- * memory at most), which the class's kernel then reads like a pump grid. */
+ * and keep the fastest (once per process and class shape); bit 1 is accepted and
+ * has no effect.  Each launch first forms, for all steps at once, the step tables of
+ * one-mode media and the pump rows of multi-mode media with a generated pump (32
+ * bytes per point and step) in a device buffer held by the batch: the classes of the
+ * largest nFreqs first, a quarter of the device memory and half of what is free at
+ * most; classes beyond that generate their pump rows in the kernel. */
 int nlm_multi_create(int n, const nlm_multi_item* items, int autotune, nlm_multi** out);
 int nlm_multi_launch(nlm_multi* batch);             /* one graph launch, asynchronous */
 int nlm_multi_sync(nlm_multi* batch, double* ms);   /* wait; ms = device time of the last launch */

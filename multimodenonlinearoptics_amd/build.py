@@ -72,9 +72,14 @@ def build(force=False, jobs=None, verbose=False):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_big.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_multi.o")
     objs.append(o)
-    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_internal.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi.hip"), "-o", o])
+    o = os.path.join(OBJ, "nlm_multi_stage.o")
+    objs.append(o)
+    deps = _deps("nlm_multi_stage.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", *dev_hdrs)
+    if force or _stale(o, deps):
+        steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi_stage.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_compose.o")
     objs.append(o)
     deps = _deps("nlm_compose.hip", "nlm_internal.hpp", *dev_hdrs)
@@ -114,7 +119,7 @@ def build(force=False, jobs=None, verbose=False):
     for m in PROP_MODELS:  # heterogeneous-batch kernels of each model
         o = os.path.join(OBJ, "nlm_multi_%d.o" % m)
         objs.append(o)
-        deps = _deps("nlm_multi_inst.hip", "nlm_multi.hpp", *dev_hdrs)
+        deps = _deps("nlm_multi_inst.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_INST_MODEL=%d" % m, "-c",
                                                 os.path.join(CSRC, "nlm_multi_inst.hip"), "-o", o])

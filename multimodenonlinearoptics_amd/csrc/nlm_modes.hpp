@@ -236,17 +236,18 @@ __device__ __forceinline__ void modes_field(const KParams& kp, F& f, cplx* field
   leave<NS>(kp, f, field, g, act, v);
 }
 
-// The power-of-two transform of one group: T = N/8 lanes, eight points each.
-template <int L, int NS>
+// The power-of-two transform of one group: T = N/8 lanes, eight points each.  ONE: a
+// workgroup holds one field however few its lanes.
+template <int L, int NS, bool ONE = false>
 struct Pow2 {
   using S = FftShape<L>;
   static constexpr int R = 8, T = S::T;
   static constexpr int ALL = NS * T;                         // lanes per field
-  static constexpr int FPB = ALL >= 64 ? 1 : 64 / ALL;       // fields per workgroup
-  static constexpr int THREADS = (FPB * ALL + 63) / 64 * 64;
+  static constexpr int FPB = ONE || ALL >= 64 ? 1 : 64 / ALL;  // fields per workgroup
+  static constexpr int THREADS = ONE && ALL < 64 ? ALL : (FPB * ALL + 63) / 64 * 64;
   static constexpr int SLOTS = (THREADS + ALL - 1) / ALL;    // the spare lanes have buffers too
   static constexpr bool WAVE = T <= 64 && 64 % T == 0;       // a group lies in one wave
-  static constexpr bool WAVE_ALL = THREADS == 64;
+  static constexpr bool WAVE_ALL = THREADS <= 64;
   // Beyond 512 lanes a wave has 128 registers: all but the first stage's twiddles come
   // from LDS, and the padding is one slot per 32 elements so that both fit.
   static constexpr bool LEAN = THREADS > 512;
@@ -282,9 +283,9 @@ struct Pow2 {
 
 // Field slot, group and lane of this thread, the twiddles and the LDS buffers of F
 // (lds: SLOTS * NS * BUF elements, then the twiddles of LEAN); returns the field's buffers.
-template <int L, int NS>
-__device__ __forceinline__ cplx* place(Pow2<L, NS>& f, cplx* lds, const cplx* tw, int* slot, int* g) {
-  using F = Pow2<L, NS>;
+template <int L, int NS, bool ONE>
+__device__ __forceinline__ cplx* place(Pow2<L, NS, ONE>& f, cplx* lds, const cplx* tw, int* slot, int* g) {
+  using F = Pow2<L, NS, ONE>;
   int s = threadIdx.x / F::ALL;
   const int r = threadIdx.x - s * F::ALL;
   int gg = r / F::T;
@@ -319,7 +320,7 @@ __global__ void __launch_bounds__((Pow2<L, M::NS>::THREADS), (ModesWaves<M, L>::
   __shared__ cplx lds[F::LDS_BYTES / sizeof(cplx)];
   F f;
   int slot, g;
-  cplx* fieldBuf = place<L, M::NS>(f, lds, kp.tw, &slot, &g);
+  cplx* fieldBuf = place(f, lds, kp.tw, &slot, &g);
   const int field = blockIdx.x * F::FPB + slot;
   modes_field<M>(kp, f, fieldBuf, field, g, slot < F::FPB && field < kp.nFields);
 }

@@ -7,12 +7,14 @@
 // (model, log2 N); every class runs as one persistent kernel whose workgroups
 // take instances from a device work queue (one atomic counter per class) in
 // order of decreasing nZ, so long propagations start first and short ones fill
-// the tail.  For media with a single linear pump the pump rows are generated
-// inside the kernel (InlinePump), so no (2nZ-1) x N pump grid is written or
-// read per instance; Chi3 (nonlinear pump) and Chi2SFGOPA (two pumps) read their
-// plan's device pump grids.  Every solver has a kernel (Chi3GNLSE with its
-// transforms inside the RK stages).  All classes are captured into one hipGraph (one branch
-// per class on its own stream, joined at the end); nlm_multi_launch replays it.
+// the tail.  What a medium's pump contributes is formed before the propagations, for
+// all steps at once (nlm_multi_stage.hip): the step tables of one-mode media, the
+// pump rows of multi-mode media with a linear pump; media whose tables or rows do not
+// fit in memory generate their rows inside the kernel (InlinePump).  Chi3 (nonlinear
+// pump) and Chi2SFGOPA (two pumps) start from their plan's device pump grids.  Every
+// solver has a kernel (Chi3GNLSE with its transforms inside the RK stages).
+// Everything is captured into one hipGraph (staging, then the classes on four
+// chains); nlm_multi_launch replays it.
 //
 // The number of persistent workgroups of a class is chosen by a small
 // autotuner at creation: each class is timed alone for a few grid sizes and
@@ -33,101 +35,35 @@ __global__ void k_zero_ints(int* p, int n) {
   if (k < n) p[k] = 0;
 }
 
-// Staged pump rows.  From N = 4096 a field's 512 lanes have 256 registers each,
-// and a propagation that generates its pump rows (InlinePump: the envelope's
-// spectrum and the running phases held per lane, two inverse transforms per
-// step) spills to scratch.  Such a class instead starts with this kernel, which
-// writes every instance's time-domain pump rows (src/_NonlinearMedium.cpp:
-// 225-250: row 0 the envelope, row r > 0 IFFT(FFT(envelope) exp(i r dzp D_p)),
-// each times the beam-profile factor) into a buffer that the class's
-// propagation kernel then reads like a medium's pump grid.  One workgroup per
-// chunk of ROWS_CHUNK rows of one instance (chunks[2b] = instance, chunks[2b+1]
-// = first row); every workgroup transforms the envelope once.
-constexpr int ROWS_L = 12;        // sizes that stage their pump rows
-constexpr int ROWS_CHUNK = 32;    // rows per workgroup
-
-template <int L>
-__global__ void __launch_bounds__(FftShape<L>::T)
-    k_multi_rows(const MultiInst* __restrict__ inst, const int* __restrict__ chunks, const cplx* __restrict__ twt) {
-  using F = FftShape<L>;
-  constexpr int N = F::N, T = F::T;
-  __shared__ cplx lds[F::lds_elems];
-  __shared__ cplx twl[PropTw<L>::LDS_ELEMS];
-  fill_twiddle_lds<L>(twl, twt);
-  const int t = threadIdx.x;
-  const MultiInst& I = inst[chunks[2 * blockIdx.x]];
-  const int r0 = chunks[2 * blockIdx.x + 1];
-  const int nZP = 2 * I.nZ - 1;
-  const int r1 = r0 + ROWS_CHUNK < nZP ? r0 + ROWS_CHUNK : nZP;
-  cplx* rows = const_cast<cplx*>(I.pump0);
-  typename PropTw<L>::type tw;
-  init_twiddles<L>(tw, twt, twl, t);
-  cplx f0[8];
-#pragma unroll
-  for (int m = 0; m < 8; m++) f0[m] = I.env[t + T * m];
-  if (r0 == 0) {
-    const double s0 = I.strength ? I.strength[0] : 1.0;
-#pragma unroll
-    for (int m = 0; m < 8; m++) rows[t + T * m] = s0 * f0[m];
-  }
-  fft_field1<L, false>(f0, lds, t, tw);
-  // the phase exp(i r dzp D_p): exact at the chunk's first row, then advanced by
-  // exp(i dzp D_p) per row (as the in-kernel generator does between its exact
-  // re-evaluations)
-  const int rb = r0 > 0 ? r0 : 1;
-  cplx ph[8], e1[8];
-#pragma unroll
-  for (int m = 0; m < 8; m++) {
-    const double d = I.Dp[t + T * m];
-    double sn, cs;
-    sincos_reduced((double)rb * I.dzp * d, &sn, &cs);
-    ph[m] = mk(cs, sn);
-    sincos_reduced(I.dzp * d, &sn, &cs);
-    e1[m] = mk(cs, sn);
-  }
-  for (int r = rb; r < r1; r++) {
-    cplx f[8];
-#pragma unroll
-    for (int m = 0; m < 8; m++) {
-      if (r > rb) ph[m] = ph[m] * e1[m];
-      f[m] = f0[m] * ph[m];
-    }
-    fft_field1<L, true>(f, lds, t, tw);
-    const double sc = (I.strength ? I.strength[r] : 1.0) * (1.0 / N);
-#pragma unroll
-    for (int m = 0; m < 8; m++) rows[(size_t)r * N + t + T * m] = f[m] * sc;
-  }
-}
-
 // Kernel of a class: models sharing a right-hand side share kernels (Chi2AFC
 // runs Chi2SFG's, Chi2ASHG Chi2SHG's).
 static int class_model(int model) {
   return model == NLM_CHI2AFC ? NLM_CHI2SFG : model == NLM_CHI2ASHG ? NLM_CHI2SHG : model;
 }
 
-static multi_fn pick_multi(int model, int L, bool inl) {
+static multi_fn pick_multi(int model, int L, int form) {
   switch (class_model(model)) {
-    case NLM_CHI3: return nlm_pick_multi_0(L, inl);
-    case NLM_CHI2PDC: return nlm_pick_multi_1(L, inl);
-    case NLM_CHI2SFG: return nlm_pick_multi_2(L, inl);
-    case NLM_CHI2SFGPDC: return nlm_pick_multi_4(L, inl);
-    case NLM_CHI2SFGII: return nlm_pick_multi_5(L, inl);
-    case NLM_CHI2PDCII: return nlm_pick_multi_6(L, inl);
-    case NLM_CHI2SFGOPA: return nlm_pick_multi_7(L, inl);
-    case NLM_CHI2SFGXPM: return nlm_pick_multi_8(L, inl);
-    case NLM_CHI2SHG: return nlm_pick_multi_9(L, inl);
-    case NLM_CHI2SHGOPA: return nlm_pick_multi_10(L, inl);
-    case NLM_CHI2DSFG: return nlm_pick_multi_11(L, inl);
-    case NLM_CHI2SHGXPM: return nlm_pick_multi_12(L, inl);
-    case NLM_CHI3GNLSE: return nlm_pick_multi_14(L, inl);
+    case NLM_CHI3: return nlm_pick_multi_0(L, form);
+    case NLM_CHI2PDC: return nlm_pick_multi_1(L, form);
+    case NLM_CHI2SFG: return nlm_pick_multi_2(L, form);
+    case NLM_CHI2SFGPDC: return nlm_pick_multi_4(L, form);
+    case NLM_CHI2SFGII: return nlm_pick_multi_5(L, form);
+    case NLM_CHI2PDCII: return nlm_pick_multi_6(L, form);
+    case NLM_CHI2SFGOPA: return nlm_pick_multi_7(L, form);
+    case NLM_CHI2SFGXPM: return nlm_pick_multi_8(L, form);
+    case NLM_CHI2SHG: return nlm_pick_multi_9(L, form);
+    case NLM_CHI2SHGOPA: return nlm_pick_multi_10(L, form);
+    case NLM_CHI2DSFG: return nlm_pick_multi_11(L, form);
+    case NLM_CHI2SHGXPM: return nlm_pick_multi_12(L, form);
+    case NLM_CHI3GNLSE: return nlm_pick_multi_14(L, form);
   }
   return nullptr;
 }
 
 struct MultiClass {
   int model, L, count, grid;
-  bool inl;   // pump rows generated in the kernel
-  bool rows;  // pump rows staged by k_multi_rows before the propagation kernel
+  int form;         // MULTI_FIELD, MULTI_INLINE, MULTI_MODES or MULTI_TAB
+  int stage;        // STAGE_*: what is formed before the propagation kernel
   int chunkOff = 0, nChunks = 0;
   multi_fn fn;
   size_t orderOff;  // offset of this class's instance order in the order array
@@ -143,8 +79,8 @@ struct nlm_multi_s {
   DevBuf<double> realBuf;
   DevBuf<MultiInst> inst;
   DevBuf<int> order, counters;
-  DevBuf<cplx> rowsBuf;  // staged pump rows of the classes with MultiClass::rows
-  DevBuf<int> chunks;    // their generation chunks (instance, first row)
+  DevBuf<cplx> stageBuf;  // step tables and pump rows of the staged classes
+  DevBuf<int> chunks;     // their chunks (instance, first step)
   std::vector<MultiClass> classes;
   hipStream_t stream = nullptr;
   hipEvent_t fork = nullptr, t0 = nullptr, t1 = nullptr;
@@ -154,7 +90,7 @@ struct nlm_multi_s {
 };
 
 static std::mutex g_tune_mu;
-static std::map<std::tuple<int, int, int, int>, int> g_tuned;  // (model, L, generated pump, count) -> grid
+static std::map<std::tuple<int, int, int, int>, int> g_tuned;  // (model, L, form, count) -> grid
 
 static int device_cus() {
   int dev = 0, cus = 256;
@@ -162,14 +98,12 @@ static int device_cus() {
   return cus > 0 ? cus : 256;
 }
 
-static void launch_rows(nlm_multi_s* m, const MultiClass& c, const cplx* tw, hipStream_t s) {
-  if (c.rows && c.nChunks > 0)
-    hipLaunchKernelGGL((k_multi_rows<ROWS_L>), dim3(c.nChunks), dim3(FftShape<ROWS_L>::T), 0, s, m->inst.p,
-                       m->chunks.p + 2 * (size_t)c.chunkOff, tw);
+static void launch_stage(nlm_multi_s* m, const MultiClass& c, const cplx* tw, hipStream_t s) {
+  nlm_multi_stage(c.stage, c.model, c.L, m->inst.p, m->chunks.p + 2 * (size_t)c.chunkOff, c.nChunks, tw, s);
 }
 
 static int run_class(nlm_multi_s* m, const MultiClass& c, int grid, const cplx* tw, hipStream_t s) {
-  launch_rows(m, c, tw, s);
+  launch_stage(m, c, tw, s);
   hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, s, m->counters.p + (&c - m->classes.data()), 1);
   c.fn(m->inst.p, m->order.p + c.orderOff, c.count, m->counters.p + (&c - m->classes.data()), tw, grid, s);
   HIP_TRY(hipGetLastError());
@@ -196,8 +130,7 @@ extern "C" int nlm_multi_destroy(nlm_multi* m) {
 extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune, nlm_multi** out) {
   if (!out || n < 0 || (n > 0 && !items)) return set_err(NLM_INVALID_ARGUMENT, "invalid arguments");
   *out = nullptr;
-  const bool stage = (autotune & 2) != 0;
-  autotune &= 1;
+  autotune &= 1;  // bit 1 (stage the pump rows) is accepted; staging is the rule below
   nlm_multi_s* m = new nlm_multi_s();
   auto fail = [&](int code) {
     nlm_multi_destroy(m);
@@ -225,7 +158,7 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
       return fail(set_err(NLM_INVALID_ARGUMENT,
                           "a pump generated in the batch needs a single linear pump; pass no envelope and run the "
                           "medium's pump simulation instead"));
-    if (!pick_multi(p->model, p->L, inl))
+    if (!pick_multi(p->model, p->L, inl ? MULTI_INLINE : MULTI_FIELD) && !pick_multi(p->model, p->L, MULTI_MODES))
       return fail(set_err(NLM_INVALID_ARGUMENT, "heterogeneous batches take nFreqs a power of two, 32..4096"));
     if (!it.input || it.cols <= 0 || it.cols % p->N != 0 || it.cols / p->N > p->nS)
       return fail(set_err(NLM_INVALID_ARGUMENT, "Signals not of correct length!"));
@@ -302,58 +235,71 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
       d.dzp = it.dzp;
     }
   }
-  // classes that stage their pump rows: ROWS_L with a generated pump (key 2),
-  // when all their rows fit a quarter of the device memory and half of what is
-  // free.  (Staging only the longer half of such a class, the shorter half
-  // generating its rows in the kernel from the start, was slower: 211 against
-  // 197 ms on 2000 SHG / PDC media.)
-  if (stage) {
-    std::vector<std::tuple<int, int, int>> keys;
-    for (auto& kv : byClass)
-      if (std::get<2>(kv.first) == 1 && std::get<1>(kv.first) == ROWS_L) keys.push_back(kv.first);
-    for (const auto& k : keys) {
-      byClass[std::make_tuple(std::get<0>(k), ROWS_L, 2)] = byClass[k];
-      byClass.erase(k);
-    }
-  }
-  if ((e = m->counters.ensure(byClass.size() + 1))) return fail(e);
-  size_t rowsTot = 0;
-  for (auto& kv : byClass)
-    if (std::get<2>(kv.first) == 2)
-      for (int i : kv.second) rowsTot += (2 * (size_t)hi[i].nZ - 1) * m->N[i];
-  bool useRows = rowsTot > 0;
-  if (useRows) {
-    size_t freeB = 0, totalB = 0;
-    useRows = hipMemGetInfo(&freeB, &totalB) == hipSuccess && rowsTot * sizeof(cplx) <= totalB / 4 &&
-              rowsTot * sizeof(cplx) <= freeB / 2;
-    if (useRows && (e = m->rowsBuf.ensure(rowsTot))) return fail(e);
-  }
-  std::vector<int> hchunks;
-  size_t rowsOff = 0;
-  // classes and their longest-first orders
-  std::vector<int> hord;
-  hord.reserve(n);
+  // What each class stages, the largest fields first (they are the longest chains and
+  // gain most) while everything staged fits a quarter of the device memory and half
+  // of what is free: the step table of one-mode media (32 bytes per point and step), or
+  // the pump rows of multi-mode media with a generated pump (as many bytes).  A class
+  // that does not fit generates its rows in the kernel, or reads its grids.
+  // SHG / PDC media of nFreqs 256..4096, nZSteps 200..4000, launch ms with every class
+  // generating its rows and the modes sharing lanes -> now: 2000 media 156 -> 132 (the
+  // N = 4096 tables take 54 GB of the budget, the other classes generate theirs), 500
+  // media 149 -> 68 (all staged, 27 GB).
+  std::vector<MultiClass> cls;
+  std::vector<std::vector<int>> members;
+  size_t freeB = 0, totalB = 0;
+  if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) freeB = totalB = 0;
+  size_t budget = std::min(totalB / 4, freeB / 2), stageTot = 0;
   for (auto& kv : byClass) {
     MultiClass c;
     c.model = std::get<0>(kv.first);
     c.L = std::get<1>(kv.first);
-    c.inl = std::get<2>(kv.first) != 0;
-    c.rows = useRows && std::get<2>(kv.first) == 2;
-    c.fn = pick_multi(c.model, c.L, c.inl && !c.rows);
-    if (c.rows) {
+    const bool groups = pick_multi(c.model, c.L, MULTI_MODES) != nullptr;
+    c.stage = STAGE_NONE;
+    c.form = std::get<2>(kv.first) ? MULTI_INLINE : groups ? MULTI_MODES : MULTI_FIELD;
+    cls.push_back(c);
+    members.push_back(kv.second);
+  }
+  std::vector<int> bySize(cls.size());
+  for (size_t k = 0; k < cls.size(); k++) bySize[k] = (int)k;
+  std::stable_sort(bySize.begin(), bySize.end(), [&](int a, int b) { return cls[a].L > cls[b].L; });
+  for (int k : bySize) {
+    MultiClass& c = cls[k];
+    const bool inl = c.form == MULTI_INLINE, table = pick_multi(c.model, c.L, MULTI_TAB) != nullptr;
+    if (!table && !(inl && pick_multi(c.model, c.L, MULTI_MODES))) continue;
+    size_t need = 0;
+    for (int i : members[k]) need += (size_t)2 * hi[i].nZ * m->N[i];
+    if (need * sizeof(cplx) > budget) continue;
+    budget -= need * sizeof(cplx);
+    stageTot += need;
+    c.stage = !table ? STAGE_ROWS : inl ? STAGE_TAB : STAGE_TAB_GRID;
+    c.form = table ? MULTI_TAB : MULTI_MODES;
+  }
+  for (auto& c : cls) {
+    c.fn = pick_multi(c.model, c.L, c.form);
+    if (!c.fn) return fail(set_err(NLM_INVALID_ARGUMENT, "heterogeneous batches take nFreqs a power of two, 32..4096"));
+  }
+  if ((e = m->counters.ensure(cls.size() + 1)) || (e = m->stageBuf.ensure(stageTot))) return fail(e);
+  std::vector<int> hchunks;
+  size_t stageOff = 0;
+  // the classes' longest-first orders
+  std::vector<int> hord;
+  hord.reserve(n);
+  for (size_t k = 0; k < cls.size(); k++) {
+    MultiClass c = cls[k];
+    if (c.stage != STAGE_NONE) {
       c.chunkOff = (int)(hchunks.size() / 2);
-      for (int i : kv.second) {
-        hi[i].pump0 = m->rowsBuf.p + rowsOff;
-        const int nZP = 2 * hi[i].nZ - 1;
-        rowsOff += (size_t)nZP * m->N[i];
-        for (int r = 0; r < nZP; r += ROWS_CHUNK) {
+      for (int i : members[k]) {
+        if (c.stage == STAGE_ROWS) hi[i].pump0 = m->stageBuf.p + stageOff;
+        else hi[i].tab = m->stageBuf.p + stageOff;
+        stageOff += (size_t)2 * hi[i].nZ * m->N[i];
+        for (int s = 1; s < hi[i].nZ || s == 1; s += MULTI_CHUNK) {
           hchunks.push_back(i);
-          hchunks.push_back(r);
+          hchunks.push_back(s);
         }
       }
       c.nChunks = (int)(hchunks.size() / 2) - c.chunkOff;
     }
-    std::vector<int> idx = kv.second;
+    std::vector<int> idx = members[k];
     std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return hi[a].nZ > hi[b].nZ; });
     c.orderOff = hord.size();
     hord.insert(hord.end(), idx.begin(), idx.end());
@@ -381,7 +327,7 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
     if ((e = get_twiddles(1 << c.L, &tw))) return fail(e);
     const int cand[4] = {cus, 2 * cus, 4 * cus, 8 * cus};
     int best = std::min(c.count, 4 * cus);
-    const auto key = std::make_tuple(c.model, c.L, c.rows ? 2 : c.inl ? 1 : 0, c.count);
+    const auto key = std::make_tuple(c.model, c.L, c.form, c.count);
     bool cached = false;
     {
       std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -417,23 +363,54 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
       return fail(set_err(NLM_DEVICE_ERROR, "stream/event creation failed"));
   }
 
-  // capture: fork one branch per class, join on the main stream
+  // Capture on at most four chains, one per hardware queue (a process has four, and
+  // work of streams that share one runs in order anyway): the classes by decreasing
+  // estimated time, each appended, its staging first, to the chain that is free first,
+  // so that the longest propagations start at once.  No chain waits for another: with
+  // the staging in a chain of its own and the staged classes waiting for it, the
+  // graph's branches were put on the queues in another order and the longest class
+  // started last (500 SHG / PDC media 127 ms).
   if (!m->classes.empty()) {
+    constexpr int CHAINS = 4;
+    const int nc = (int)m->classes.size(), chains = std::min(CHAINS, nc);
+    std::vector<int> byCost(nc);
+    std::vector<double> cost(nc);
+    for (int k = 0; k < nc; k++) {
+      const MultiClass& c = m->classes[k];
+      byCost[k] = k;
+      // microseconds per step of one propagation beside others: step-table classes, and
+      // the others (several modes or transforms per step); staging writes 32 bytes per
+      // point and step at ~2 TB/s
+      static const double tabUs[8] = {1.6, 1.6, 1.6, 1.6, 2.0, 2.4, 4.6, 7.4};
+      static const double otherUs[8] = {3.2, 3.2, 3.2, 3.2, 3.2, 6.0, 8.0, 14.0};
+      cost[k] = (c.form == MULTI_TAB ? tabUs : otherUs)[c.L - 5] * hi[hord[c.orderOff]].nZ;
+      if (c.stage != STAGE_NONE)
+        for (int j = 0; j < c.count; j++) cost[k] += hi[hord[c.orderOff + j]].nZ * (double)(1 << c.L) * 1.6e-5;
+    }
+    std::stable_sort(byCost.begin(), byCost.end(), [&](int a, int b) { return cost[a] > cost[b]; });
+    double load[CHAINS] = {0, 0, 0, 0};
     HIP_TRY(hipStreamBeginCapture(m->stream, hipStreamCaptureModeThreadLocal));
-    hipError_t ce = hipEventRecord(m->fork, m->stream);
-    for (auto& c : m->classes) {
+    hipLaunchKernelGGL(k_zero_ints, dim3((nc + 255) / 256), dim3(256), 0, m->stream, m->counters.p, nc);
+    hipError_t ce = hipGetLastError();
+    if (ce == hipSuccess) ce = hipEventRecord(m->fork, m->stream);
+    for (int q = 0; q < chains && ce == hipSuccess; q++) ce = hipStreamWaitEvent(m->classes[q].stream, m->fork, 0);
+    for (int k : byCost) {
+      if (ce != hipSuccess) break;
+      const MultiClass& c = m->classes[k];
+      int q = 0;
+      for (int j = 1; j < chains; j++)
+        if (load[j] < load[q]) q = j;
+      load[q] += cost[k];
+      hipStream_t s = m->classes[q].stream;
       const cplx* tw = nullptr;
       (void)get_twiddles(1 << c.L, &tw);
-      if (ce == hipSuccess) ce = hipStreamWaitEvent(c.stream, m->fork, 0);
-      if (ce == hipSuccess) {
-        launch_rows(m, c, tw, c.stream);
-        hipLaunchKernelGGL(k_zero_ints, dim3(1), dim3(64), 0, c.stream, m->counters.p + (&c - m->classes.data()), 1);
-        c.fn(m->inst.p, m->order.p + c.orderOff, c.count, m->counters.p + (&c - m->classes.data()), tw, c.grid,
-             c.stream);
-        ce = hipGetLastError();
-      }
-      if (ce == hipSuccess) ce = hipEventRecord(c.done, c.stream);
-      if (ce == hipSuccess) ce = hipStreamWaitEvent(m->stream, c.done, 0);
+      launch_stage(m, c, tw, s);
+      c.fn(m->inst.p, m->order.p + c.orderOff, c.count, m->counters.p + k, tw, c.grid, s);
+      ce = hipGetLastError();
+    }
+    for (int q = 0; q < chains && ce == hipSuccess; q++) {
+      ce = hipEventRecord(m->classes[q].done, m->classes[q].stream);
+      if (ce == hipSuccess) ce = hipStreamWaitEvent(m->stream, m->classes[q].done, 0);
     }
     hipGraph_t g = nullptr;
     hipError_t ee = hipStreamEndCapture(m->stream, &g);

@@ -11,28 +11,51 @@
 
 namespace {
 using MM = typename ModelOf<NLM_INST_MODEL>::type;
+constexpr bool GNLSE = NLM_INST_MODEL == NLM_CHI3GNLSE;
 // the pump rows can be generated in the kernel for a single linear pump
 // (_NonlinearMedium::runPumpSimulation); Chi3's pump is nonlinear (solvers/Chi3.cpp:25-54)
-constexpr bool CAN_INLINE = MM::NP == 1 && NLM_INST_MODEL != NLM_CHI3;
+constexpr bool LINEAR = MM::NP == 1 && NLM_INST_MODEL != NLM_CHI3;
+// media with a step table (R-linear, one mode): Chi3 and Chi2PDC
+constexpr bool TABLE = MM::NS == 1 && MM::NP == 1;
 
-template <bool INL>
+template <int L, int FORM>
+constexpr bool has() {
+  if constexpr (FORM == MULTI_MODES) return MM::NS > 1 && modes::Pow2<L, MM::NS, true>::OK;
+  else if constexpr (FORM == MULTI_TAB) return TABLE;
+  else if constexpr (FORM == MULTI_INLINE) return LINEAR;
+  // lanes shared by all modes: media without a generated pump where the mode groups
+  // do not fit, and one-mode media whose table was not staged
+  else return GNLSE || TABLE || (MM::NS > 1 && !modes::Pow2<L, MM::NS, true>::OK);
+}
+
+template <int L, int FORM>
+multi_fn one() {
+  if constexpr (has<L, FORM>()) return &launch_multi<MM, L, FORM>;
+  else return nullptr;
+}
+
+template <int FORM>
 multi_fn pick(int L) {
-  if constexpr (INL && !CAN_INLINE) {
-    return nullptr;
-  } else {
-    switch (L) {
-      case 5: return &launch_multi<MM, 5, INL>;
-      case 6: return &launch_multi<MM, 6, INL>;
-      case 7: return &launch_multi<MM, 7, INL>;
-      case 8: return &launch_multi<MM, 8, INL>;
-      case 9: return &launch_multi<MM, 9, INL>;
-      case 10: return &launch_multi<MM, 10, INL>;
-      case 11: return &launch_multi<MM, 11, INL>;
-      case 12: return &launch_multi<MM, 12, INL>;
-    }
-    return nullptr;
+  switch (L) {
+    case 5: return one<5, FORM>();
+    case 6: return one<6, FORM>();
+    case 7: return one<7, FORM>();
+    case 8: return one<8, FORM>();
+    case 9: return one<9, FORM>();
+    case 10: return one<10, FORM>();
+    case 11: return one<11, FORM>();
+    case 12: return one<12, FORM>();
   }
+  return nullptr;
 }
 }  // namespace
 
-multi_fn NLM_CAT(nlm_pick_multi_, NLM_INST_MODEL)(int L, bool inl) { return inl ? pick<true>(L) : pick<false>(L); }
+multi_fn NLM_CAT(nlm_pick_multi_, NLM_INST_MODEL)(int L, int form) {
+  switch (form) {
+    case MULTI_FIELD: return pick<MULTI_FIELD>(L);
+    case MULTI_INLINE: return pick<MULTI_INLINE>(L);
+    case MULTI_MODES: return pick<MULTI_MODES>(L);
+    case MULTI_TAB: return pick<MULTI_TAB>(L);
+  }
+  return nullptr;
+}

@@ -18,6 +18,39 @@ __device__ __forceinline__ cplx rk4_step(const cplx* c, const cplx* cc, cplx x, 
   return x + (((k1[0] + 2.0 * k2[0]) + 2.0 * k3[0]) + k4[0]) * (1. / 6.);
 }
 
+// The RK4 step as a real 2 x 2 matrix on (Re x, Im x), times s: columns R(1) and R(i),
+// row p = (Re R(1), Re R(i)), row q = (Im R(1), Im R(i)).
+template <class M>
+struct StepMatrix {
+  static __device__ __forceinline__ void eval(const cplx* c, const cplx* cc, cplx P0, cplx P1, cplx P2, double s,
+                                              cplx& p, cplx& q) {
+    const cplx a = rk4_step<M>(c, cc, mk(1.0, 0.0), P0, P1, P2);
+    const cplx b = rk4_step<M>(c, cc, mk(0.0, 1.0), P0, P1, P2);
+    p = mk(s * a.re, s * b.re);
+    q = mk(s * a.im, s * b.im);
+  }
+};
+
+// Chi2PDC: k(x) = m conj(x) with m1, m2, m3 = c P at the three positions, so the RK4
+// stages expand to x' = alpha x + beta conj(x),
+//   alpha = 1 + (m2 conj(m1) + |m2|^2 + m3 conj(q)) / 6,
+//   beta = (m1 + 2 m2 + 2 q + (1 + |m2|^2 / 2) m3) / 6,   q = m2 + |m2|^2 m1 / 4:
+// ~45 FP64 operations instead of two RK4 steps' ~120.
+template <>
+struct StepMatrix<MChi2PDC> {
+  static __device__ __forceinline__ void eval(const cplx* c, const cplx*, cplx P0, cplx P1, cplx P2, double s, cplx& p,
+                                              cplx& q) {
+    const cplx m1 = c[0] * P0, m2 = c[1] * P1, m3 = c[2] * P2;
+    const double n = abs2(m2);
+    const cplx r = m2 + (0.25 * n) * m1;
+    const cplx u = m2 * conj(m1) + m3 * conj(r);
+    const cplx be = (m1 + 2.0 * (m2 + r) + (1.0 + 0.5 * n) * m3) * (1. / 6.);
+    const double ar = 1.0 + (u.re + n) * (1. / 6.), ai = u.im * (1. / 6.);
+    p = mk(s * (ar + be.re), s * (be.im - ai));
+    q = mk(s * (ai + be.im), s * (ar - be.re));
+  }
+};
+
 template <int L>
 __device__ __forceinline__ void load_prop_row(cplx (&al)[8], cplx (&be)[8], const cplx* __restrict__ row, int t) {
   constexpr int T = FftShape<L>::T;
