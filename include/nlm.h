@@ -246,6 +246,20 @@ int nlm_greens_forward(nlm_plan* plan, int in_time_domain, int n_in, const int32
 int nlm_greens_adjoint(nlm_plan* plan, const double* gC, const double* gS, double* g_coef, double* g_pump_time,
                        double* g_envelope);
 
+/* Nonzero where ptr is memory of the plan's device known to this process's HIP
+ * runtime (a process can hold two, whose allocations are not each other's). */
+int nlm_plan_owns_device_of(nlm_plan* plan, const void* ptr);
+
+/* The same with matrices in device memory of the plan's device (one mode; C_dev,
+ * S_dev, gC_dev, gS_dev: N x N complex): nothing but g_coef ([nZ][3] complex) and
+ * g_envelope ([N] complex, or NULL) crosses to the host.  The caller's work on these
+ * buffers must be complete; both calls return when theirs is.  Memory that is not of
+ * the plan's device, or not known to this process's HIP runtime, is refused with
+ * NLM_INVALID_ARGUMENT. */
+int nlm_greens_forward_dev(nlm_plan* plan, int in_time_domain, int ckpt_every, double* C_dev, double* S_dev);
+int nlm_greens_adjoint_dev(nlm_plan* plan, const double* gC_dev, const double* gS_dev, double* g_coef,
+                           double* g_envelope);
+
 /* Differentiable Chi3GNLSE batch (batchSignalSimulation of a fully nonlinear
  * medium, src/_FullyNonlinearMedium.hpp:8-11 with Chi3GNLSE::DiffEq,
  * solvers/Chi3GNLSE.cpp:39-92, inside signalSimulationTemplate,
@@ -262,6 +276,11 @@ int nlm_greens_adjoint(nlm_plan* plan, const double* gC, const double* gS, doubl
 int nlm_batch_forward(nlm_plan* plan, const double* inputs, int rows, int in_time_domain, int ckpt_every,
                       double* out);
 int nlm_batch_adjoint(nlm_plan* plan, const double* g_out, double* g_in);
+/* The same with every array in device memory of the plan's device (as
+ * nlm_greens_forward_dev). */
+int nlm_batch_forward_dev(nlm_plan* plan, const double* inputs_dev, int rows, int in_time_domain, int ckpt_every,
+                          double* out_dev);
+int nlm_batch_adjoint_dev(nlm_plan* plan, const double* g_out_dev, double* g_in_dev);
 
 /* Green's function composition of two media, Cascade::computeGreensFunction
  * (src/Cascade.cpp:128-129): C = C2 C1 + S2 conj(S1), S = C2 S1 + S2 conj(C1).

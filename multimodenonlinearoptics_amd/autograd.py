@@ -29,6 +29,23 @@ def _check_serial(ctx):
                            "per graph")
 
 
+def _plain(t):
+    """t as a detached contiguous complex128 tensor without lazy conjugation or negation,
+    so that its memory holds its values."""
+    return t.detach().to(torch.complex128).resolve_conj().resolve_neg().contiguous()
+
+
+def _direct(medium, *tensors):
+    """Whether the engine can work on the tensors' own memory: complex128 matrices on the
+    medium's device, allocated by the HIP runtime that the engine runs on (a process
+    can hold two: torch's own and the system's).  Waits for the pending work on them if so: the
+    engine runs on the medium's stream."""
+    if not all(t.is_cuda for t in tensors) or not medium.onDevice([t.data_ptr() for t in tensors]):
+        return False
+    torch.cuda.current_stream(tensors[0].device).synchronize()
+    return True
+
+
 class GreensFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, medium, envelope, poling, ckpt_every=0):
@@ -36,41 +53,55 @@ class GreensFunction(torch.autograd.Function):
         pol = poling.detach().cpu().numpy().astype(np.float64)
         medium.setPump(env)
         medium.setPolingProfile(pol)
-        C, S = medium.greensForward(False, True, int(ckpt_every))
+        n = len(medium.omega)
+        C, S = (torch.empty((n, n), dtype=torch.complex128, device=envelope.device) for _ in range(2))
+        if _direct(medium, C, S):
+            medium.greensForwardDev(C.data_ptr(), S.data_ptr(), False, True, int(ckpt_every))
+        else:
+            C, S = (torch.from_numpy(a).to(envelope.device) for a in medium.greensForward(False, True, int(ckpt_every)))
         ctx.medium = medium
         ctx.serial = medium.forwardSerial
         ctx.device = envelope.device
-        return torch.from_numpy(C).to(envelope.device), torch.from_numpy(S).to(envelope.device)
+        return C, S
 
     @staticmethod
     def backward(ctx, gC, gS):
         _check_serial(ctx)
-        gC = np.zeros(0) if gC is None else gC.detach().cpu().numpy()
-        gS = np.zeros(0) if gS is None else gS.detach().cpu().numpy()
-        n = ctx.medium.signalFreq.shape[1]
-        if gC.size == 0:
-            gC = np.zeros((n, n), dtype=np.complex128)
-        if gS.size == 0:
-            gS = np.zeros((n, n), dtype=np.complex128)
-        g_env, g_pol = ctx.medium.greensAdjoint(gC.astype(np.complex128), gS.astype(np.complex128))
+        n = len(ctx.medium.omega)
+        gC, gS = (torch.zeros((n, n), dtype=torch.complex128, device=ctx.device) if g is None else _plain(g)
+                  for g in (gC, gS))
+        if gC.shape == gS.shape == (n, n) and _direct(ctx.medium, gC, gS):
+            g_env, g_pol = ctx.medium.greensAdjointDev(gC.data_ptr(), gS.data_ptr())
+        else:
+            g_env, g_pol = ctx.medium.greensAdjoint(gC.cpu().numpy(), gS.cpu().numpy())
         return (None, torch.from_numpy(g_env).to(ctx.device), torch.from_numpy(g_pol).to(ctx.device), None)
 
 
 class BatchSignal(torch.autograd.Function):
     @staticmethod
     def forward(ctx, medium, inputs, inTimeDomain=True, ckpt_every=0):
-        x = inputs.detach().cpu().numpy().astype(np.complex128)
-        out = medium.batchForward(x, bool(inTimeDomain), int(ckpt_every))
+        x = _plain(inputs)
+        out = torch.empty_like(x)
+        if x.dim() == 2 and x.shape[0] > 0 and x.shape[1] == len(medium.omega) and _direct(medium, x, out):
+            medium.batchForwardDev(x.data_ptr(), x.shape[0], out.data_ptr(), bool(inTimeDomain), int(ckpt_every))
+        else:
+            out = torch.from_numpy(medium.batchForward(x.cpu().numpy(), bool(inTimeDomain), int(ckpt_every)))
         ctx.medium = medium
         ctx.serial = medium.forwardSerial
         ctx.device = inputs.device
-        return torch.from_numpy(out).to(inputs.device)
+        ctx.shape = out.shape
+        return out.to(inputs.device)
 
     @staticmethod
     def backward(ctx, g):
         _check_serial(ctx)
-        gin = ctx.medium.batchAdjoint(g.detach().cpu().numpy().astype(np.complex128))
-        return None, torch.from_numpy(gin).to(ctx.device), None, None
+        g = _plain(g)
+        gin = torch.empty_like(g)
+        if g.shape == ctx.shape and _direct(ctx.medium, g, gin):
+            ctx.medium.batchAdjointDev(g.data_ptr(), gin.data_ptr())
+        else:
+            gin = torch.from_numpy(ctx.medium.batchAdjoint(g.cpu().numpy()))
+        return None, gin.to(ctx.device), None, None
 
 
 def band_energy_loss(out_time, omega, lo=5.0, hi=15.0):

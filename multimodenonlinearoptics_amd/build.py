@@ -90,6 +90,11 @@ def build(force=False, jobs=None, verbose=False):
     deps = _deps("nlm_any.hip", "nlm_mix.hpp", "nlm_modes.hpp", "nlm_internal.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_any.hip"), "-o", o])
+    o = os.path.join(OBJ, "nlm_copy.o")
+    objs.append(o)
+    deps = _deps("nlm_copy.hip", "nlm_internal.hpp", *dev_hdrs)
+    if force or _stale(o, deps):
+        steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_copy.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_noalloc.o")
     objs.append(o)
     deps = _deps("nlm_noalloc.hip", "nlm_internal.hpp", *dev_hdrs)

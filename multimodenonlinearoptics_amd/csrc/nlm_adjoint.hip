@@ -100,9 +100,21 @@ static int default_ckpt_every(const nlm_plan_s* p, size_t nF) {
   return (int)std::max<size_t>(1, std::min<size_t>(K, (size_t)kSqrt));
 }
 
-extern "C" int nlm_greens_forward(nlm_plan* p, int in_time, int n_in, const int32_t* inputs, int n_out,
-                                  const int32_t* outputs, const double* block_scale, int ckpt_every, double* C,
-                                  double* S) {
+static int to_matrices(nlm_plan* p, size_t bytes, double* C, double* S, bool dev) {
+  if (!dev) {
+    const HostCopy out[2] = {{C, p->C.p, bytes}, {S, p->S.p, bytes}};
+    return nlm_to_host(out, 2, p->stream);
+  }
+  HIP_TRY(hipMemcpyAsync(C, p->C.p, bytes, hipMemcpyDeviceToDevice, p->stream));
+  HIP_TRY(hipMemcpyAsync(S, p->S.p, bytes, hipMemcpyDeviceToDevice, p->stream));
+  HIP_TRY(hipStreamSynchronize(p->stream));
+  return NLM_OK;
+}
+
+// nlm_greens_forward, and with dev its form with C and S in device memory
+static int greens_forward(nlm_plan* p, int in_time, int n_in, const int32_t* inputs, int n_out,
+                          const int32_t* outputs, const double* block_scale, int ckpt_every, double* C, double* S,
+                          bool dev) {
   if (!p || !inputs || !outputs) return set_err(NLM_INVALID_ARGUMENT, "null argument");
   if (p->model != NLM_CHI2PDC)
     return set_err(NLM_INVALID_ARGUMENT, "the adjoint Green's function is implemented for Chi2PDC");
@@ -148,9 +160,7 @@ extern "C" int nlm_greens_forward(nlm_plan* p, int in_time, int n_in, const int3
   p->gInTime = in_time;
   p->adjGen = ++p->gen;
   (void)block_scale;
-  if (C) HIP_TRY(hipMemcpyAsync(C, p->C.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (S) HIP_TRY(hipMemcpyAsync(S, p->S.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  if (int e = to_matrices(p, total * sizeof(cplx), C, S, dev)) return e;
   if (p->timing) {
     collect_timing(p, 2, 3, 1);
     collect_timing(p, 3, 4, 2);
@@ -158,8 +168,27 @@ extern "C" int nlm_greens_forward(nlm_plan* p, int in_time, int n_in, const int3
   return NLM_OK;
 }
 
-extern "C" int nlm_greens_adjoint(nlm_plan* p, const double* gC, const double* gS, double* g_coef,
-                                  double* g_pump_time, double* g_envelope) {
+extern "C" int nlm_greens_forward(nlm_plan* p, int in_time, int n_in, const int32_t* inputs, int n_out,
+                                  const int32_t* outputs, const double* block_scale, int ckpt_every, double* C,
+                                  double* S) {
+  return greens_forward(p, in_time, n_in, inputs, n_out, outputs, block_scale, ckpt_every, C, S, false);
+}
+
+static int check_device(nlm_plan* p, const void* a, const void* b) {
+  if (!p) return set_err(NLM_INVALID_ARGUMENT, "null plan");
+  if (!nlm_on_device(a, p->device) || !nlm_on_device(b, p->device))
+    return set_err(NLM_INVALID_ARGUMENT, "not memory of the plan's device");
+  return NLM_OK;
+}
+
+extern "C" int nlm_greens_forward_dev(nlm_plan* p, int in_time, int ckpt_every, double* C_dev, double* S_dev) {
+  if (int e = check_device(p, C_dev, S_dev)) return e;
+  const int32_t m0 = 0;
+  return greens_forward(p, in_time, 1, &m0, 1, &m0, nullptr, ckpt_every, C_dev, S_dev, true);
+}
+
+static int greens_adjoint(nlm_plan* p, const double* gC, const double* gS, double* g_coef, double* g_pump_time,
+                          double* g_envelope, bool dev) {
   if (!p || !gC || !gS || !g_coef) return set_err(NLM_INVALID_ARGUMENT, "null argument");
   if (!p->nSeg || !p->ckpt.p) return set_err(NLM_RUNTIME_ERROR, "run nlm_greens_forward before the adjoint");
   if (p->adjGen != p->gen)
@@ -199,7 +228,7 @@ extern "C" int nlm_greens_adjoint(nlm_plan* p, const double* gC, const double* g
   const bool rows = g_pump_time || g_envelope;
   const int nEnv = std::min(nZP - 1 > 0 ? nZP - 1 : 1, 512);
   int e;
-  if ((e = p->gC.ensure(total)) || (e = p->gS.ensure(total)) || (e = p->gG.ensure(nF * W)) ||
+  if ((!dev && ((e = p->gC.ensure(total)) || (e = p->gS.ensure(total)))) || (e = p->gG.ensure(nF * W)) ||
       (e = p->gcoefPart.ensure((size_t)nZ * 3 * N)) || (e = p->gcoef.ensure((size_t)nZ * 3)) ||
       (e = p->stepTab.ensure((size_t)nZ * N * 2)) ||
       (e = p->gpumpPart.ensure(perStep * chunk)) || (e = p->gtmp.ensure(nF * 2 * N)))
@@ -207,10 +236,13 @@ extern "C" int nlm_greens_adjoint(nlm_plan* p, const double* gC, const double* g
   if (slices > 1 && (e = p->gslice.ensure((size_t)slices * chunk * 2 * N))) return e;
   if (rows && (e = p->gpump.ensure((size_t)nZP * N))) return e;
   if (g_envelope && ((e = p->gF0Part.ensure((size_t)nEnv * N)) || (e = p->gF0.ensure(3 * (size_t)N)))) return e;
-  HIP_TRY(hipMemcpyAsync(p->gC.p, gC, total * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
-  HIP_TRY(hipMemcpyAsync(p->gS.p, gS, total * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
+  if (!dev && ((e = nlm_to_device(p->gC.p, gC, total * sizeof(cplx), p->stream)) ||
+               (e = nlm_to_device(p->gS.p, gS, total * sizeof(cplx), p->stream))))
+    return e;
+  const cplx* gCd = dev ? reinterpret_cast<const cplx*>(gC) : p->gC.p;
+  const cplx* gSd = dev ? reinterpret_cast<const cplx*>(gS) : p->gS.p;
   hipLaunchKernelGGL(k_greens_assemble_adjoint, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, p->stream,
-                     p->gC.p, p->gS.p, p->gG.p, N, 1, 1, 1, (const cplx*)nullptr);
+                     gCd, gSd, p->gG.p, N, 1, 1, 1, (const cplx*)nullptr);
   // the step propagators (the states between checkpoints are rebuilt by inverting them)
   nlm_launch_step_table(NLM_CHI2PDC, p->coef.p, p->cconst.p, p->pumpT[0].p, N, nZ, p->stepTab.p, p->stream);
   HIP_TRY(hipGetLastError());
@@ -287,16 +319,26 @@ extern "C" int nlm_greens_adjoint(nlm_plan* p, const double* gC, const double* g
     hipLaunchKernelGGL(k_env_grad, dim3((N + 255) / 256), dim3(256), 0, p->stream, p->gF0.p + N, p->gpump.p, s0, N,
                        p->gF0.p + 2 * N);
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(g_envelope, p->gF0.p + 2 * N, N * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
   }
   tic(p, 4);
-  HIP_TRY(hipMemcpyAsync(g_coef, p->gcoef.p, (size_t)nZ * 3 * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (g_pump_time)
-    HIP_TRY(hipMemcpyAsync(g_pump_time, p->gpump.p, (size_t)nZP * N * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  const HostCopy out[3] = {{g_envelope, g_envelope ? p->gF0.p + 2 * N : nullptr, N * sizeof(cplx)},
+                           {g_coef, p->gcoef.p, (size_t)nZ * 3 * sizeof(cplx)},
+                           {g_pump_time, p->gpump.p, (size_t)nZP * N * sizeof(cplx)}};
+  if ((e = nlm_to_host(out, 3, p->stream))) return e;
   if (p->timing) {
     collect_timing(p, 2, 3, 1);
     collect_timing(p, 3, 4, 2);
   }
   return NLM_OK;
+}
+
+extern "C" int nlm_greens_adjoint(nlm_plan* p, const double* gC, const double* gS, double* g_coef,
+                                  double* g_pump_time, double* g_envelope) {
+  return greens_adjoint(p, gC, gS, g_coef, g_pump_time, g_envelope, false);
+}
+
+extern "C" int nlm_greens_adjoint_dev(nlm_plan* p, const double* gC_dev, const double* gS_dev, double* g_coef,
+                                      double* g_envelope) {
+  if (int e = check_device(p, gC_dev, gS_dev)) return e;
+  return greens_adjoint(p, gC_dev, gS_dev, g_coef, nullptr, g_envelope, true);
 }

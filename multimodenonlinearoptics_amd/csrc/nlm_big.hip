@@ -571,8 +571,40 @@ static int gnlse_diff_check(nlm_plan* p) {
   return NLM_OK;
 }
 
+// a result into the caller's host memory, or into its device memory (dev)
+static int from_device(nlm_plan* p, double* dst, const cplx* src, size_t bytes, bool dev) {
+  if (!dev) {
+    const HostCopy c = {dst, src, bytes};
+    return nlm_to_host(&c, 1, p->stream);
+  }
+  HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToDevice, p->stream));
+  HIP_TRY(hipStreamSynchronize(p->stream));
+  return NLM_OK;
+}
+
+static int batch_forward(nlm_plan* p, const double* inputs, int rows, int in_time, int ckpt_every, double* out,
+                         bool dev);
+
 extern "C" int nlm_batch_forward(nlm_plan* p, const double* inputs, int rows, int in_time, int ckpt_every,
                                  double* out) {
+  return batch_forward(p, inputs, rows, in_time, ckpt_every, out, false);
+}
+
+static int check_device(nlm_plan* p, const void* a, const void* b) {
+  if (!p) return set_err(NLM_INVALID_ARGUMENT, "null plan");
+  if (!nlm_on_device(a, p->device) || !nlm_on_device(b, p->device))
+    return set_err(NLM_INVALID_ARGUMENT, "not memory of the plan's device");
+  return NLM_OK;
+}
+
+extern "C" int nlm_batch_forward_dev(nlm_plan* p, const double* inputs_dev, int rows, int in_time, int ckpt_every,
+                                     double* out_dev) {
+  if (int e = check_device(p, inputs_dev, out_dev)) return e;
+  return batch_forward(p, inputs_dev, rows, in_time, ckpt_every, out_dev, true);
+}
+
+static int batch_forward(nlm_plan* p, const double* inputs, int rows, int in_time, int ckpt_every, double* out,
+                         bool dev) {
   if (int e = gnlse_diff_check(p)) return e;
   if (!inputs || !out || rows <= 0) return set_err(NLM_INVALID_ARGUMENT, "null argument or empty batch");
   const int N = p->N, nSteps = p->nZ - 1;
@@ -585,7 +617,8 @@ extern "C" int nlm_batch_forward(nlm_plan* p, const double* inputs, int rows, in
   const Stager sg = pick_stager(p->L);
   int e;
   if ((e = p->in.ensure(BN)) || (e = p->out.ensure(BN)) || (e = p->ckpt.ensure((size_t)nSeg * BN))) return e;
-  HIP_TRY(hipMemcpyAsync(p->in.p, inputs, BN * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
+  if (dev) HIP_TRY(hipMemcpyAsync(p->in.p, inputs, BN * sizeof(cplx), hipMemcpyDeviceToDevice, p->stream));
+  else if ((e = nlm_to_device(p->in.p, inputs, BN * sizeof(cplx), p->stream))) return e;
   BigParams bp;
   if ((e = setup_params(p, sg, rows, bp))) return e;
   bp.in = p->in.p;
@@ -604,8 +637,7 @@ extern "C" int nlm_batch_forward(nlm_plan* p, const double* inputs, int rows, in
   for (int i = 1; i <= nSteps; i++) launch_step(sg, bp, 0, i, p->stream);
   HIP_TRY(hipGetLastError());
   tic(p, 3);
-  HIP_TRY(hipMemcpyAsync(out, p->out.p, BN * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  if ((e = from_device(p, out, p->out.p, BN * sizeof(cplx), dev))) return e;
   if (p->timing) collect_timing(p, 2, 3, 1);
   p->ckptEvery = K;
   p->nSeg = nSeg;
@@ -615,7 +647,18 @@ extern "C" int nlm_batch_forward(nlm_plan* p, const double* inputs, int rows, in
   return NLM_OK;
 }
 
+static int batch_adjoint(nlm_plan* p, const double* g_out, double* g_in, bool dev);
+
 extern "C" int nlm_batch_adjoint(nlm_plan* p, const double* g_out, double* g_in) {
+  return batch_adjoint(p, g_out, g_in, false);
+}
+
+extern "C" int nlm_batch_adjoint_dev(nlm_plan* p, const double* g_out_dev, double* g_in_dev) {
+  if (int e = check_device(p, g_out_dev, g_in_dev)) return e;
+  return batch_adjoint(p, g_out_dev, g_in_dev, true);
+}
+
+static int batch_adjoint(nlm_plan* p, const double* g_out, double* g_in, bool dev) {
   if (int e = gnlse_diff_check(p)) return e;
   if (!g_out || !g_in) return set_err(NLM_INVALID_ARGUMENT, "null argument");
   if (p->bRows <= 0 || !p->nSeg || !p->ckpt.p)
@@ -631,7 +674,8 @@ extern "C" int nlm_batch_adjoint(nlm_plan* p, const double* g_out, double* g_in)
   if ((e = p->gG.ensure(BN)) || (e = p->gtmp.ensure(BN)) || (e = p->adjWork.ensure(3 * BN)) ||
       (e = p->adjSeg.ensure((size_t)8 * K * BN)))
     return e;
-  HIP_TRY(hipMemcpyAsync(p->gG.p, g_out, BN * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
+  if (dev) HIP_TRY(hipMemcpyAsync(p->gG.p, g_out, BN * sizeof(cplx), hipMemcpyDeviceToDevice, p->stream));
+  else if ((e = nlm_to_device(p->gG.p, g_out, BN * sizeof(cplx), p->stream))) return e;
   BigParams bp;
   if ((e = setup_params(p, sg, rows, bp))) return e;
   bp.inCols = N;
@@ -667,8 +711,7 @@ extern "C" int nlm_batch_adjoint(nlm_plan* p, const double* g_out, double* g_in)
   }
   HIP_TRY(hipGetLastError());
   tic(p, 3);
-  HIP_TRY(hipMemcpyAsync(g_in, p->gtmp.p, BN * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  if ((e = from_device(p, g_in, p->gtmp.p, BN * sizeof(cplx), dev))) return e;
   if (p->timing) collect_timing(p, 2, 3, 1);
   return NLM_OK;
 }

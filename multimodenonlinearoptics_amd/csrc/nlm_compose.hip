@@ -179,7 +179,8 @@ extern "C" int nlm_greens_cascade(int n, nlm_plan* const* plans, double* C, doub
   const int cols = plans[0]->greensCols;
   const cplx* aC = plans[0]->C.p;
   const cplx* aS = plans[0]->S.p;
-  DevBuf<cplx> buf[2][2];
+  // products alternate between two pairs of buffers that the last plan keeps
+  DevBuf<cplx>(&buf)[2][2] = plans[n - 1]->cascade;
   for (int i = 1; i < n; i++) {
     const int M = plans[i]->greensRows, K = plans[i]->greensCols;
     if (K != rows) return set_err(NLM_INVALID_ARGUMENT, "Green's function shapes of adjacent media do not match");
@@ -193,10 +194,8 @@ extern "C" int nlm_greens_cascade(int n, nlm_plan* const* plans, double* C, doub
     rows = M;
   }
   const size_t total = (size_t)rows * cols;
-  HIP_TRY(hipMemcpyAsync(C, aC, total * sizeof(cplx), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipMemcpyAsync(S, aS, total * sizeof(cplx), hipMemcpyDeviceToHost, s));
-  HIP_TRY(hipStreamSynchronize(s));
-  return NLM_OK;
+  const HostCopy out[2] = {{C, aC, total * sizeof(cplx)}, {S, aS, total * sizeof(cplx)}};
+  return nlm_to_host(out, 2, s);
 }
 
 // ---------------------------------------------------------------------------

@@ -420,7 +420,7 @@ extern "C" int nlm_model_ncoef(int model, int32_t* nc, int32_t* ncc, int32_t* ns
 static int upload(DevBuf<cplx>& b, const double* src, size_t count, hipStream_t s) {
   int e = b.ensure(count);
   if (e) return e;
-  if (count && src) HIP_TRY(hipMemcpyAsync(b.p, src, count * sizeof(cplx), hipMemcpyHostToDevice, s));
+  if (count && src) return nlm_to_device(b.p, src, count * sizeof(cplx), s);
   return NLM_OK;
 }
 
@@ -621,8 +621,10 @@ extern "C" int nlm_pump_upload(nlm_plan* p, int q, const double* pump_time, cons
   plan_touch(p);
   if (int e = ensure_pumps(p)) return e;
   const size_t cnt = (2 * (size_t)p->nZ - 1) * p->N;
-  if (pump_time) HIP_TRY(hipMemcpyAsync(p->pumpT[q].p, pump_time, cnt * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
-  if (pump_freq) HIP_TRY(hipMemcpyAsync(p->pumpF[q].p, pump_freq, cnt * sizeof(cplx), hipMemcpyHostToDevice, p->stream));
+  if (pump_time)
+    if (int e = nlm_to_device(p->pumpT[q].p, pump_time, cnt * sizeof(cplx), p->stream)) return e;
+  if (pump_freq)
+    if (int e = nlm_to_device(p->pumpF[q].p, pump_freq, cnt * sizeof(cplx), p->stream)) return e;
   HIP_TRY(hipStreamSynchronize(p->stream));
   p->pumpLinear = false;
   return NLM_OK;
@@ -679,10 +681,8 @@ extern "C" int nlm_pump_download(nlm_plan* p, int q, double* pump_time, double* 
   if (q < 0 || q >= p->nP) return set_err(NLM_INVALID_ARGUMENT, "Invalid pump index");
   if (!p->pumpT[q].p) return set_err(NLM_RUNTIME_ERROR, "pump grid has not been computed");
   const size_t cnt = (2 * (size_t)p->nZ - 1) * p->N;
-  if (pump_time) HIP_TRY(hipMemcpyAsync(pump_time, p->pumpT[q].p, cnt * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (pump_freq) HIP_TRY(hipMemcpyAsync(pump_freq, p->pumpF[q].p, cnt * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
-  return NLM_OK;
+  const HostCopy out[2] = {{pump_time, p->pumpT[q].p, cnt * sizeof(cplx)}, {pump_freq, p->pumpF[q].p, cnt * sizeof(cplx)}};
+  return nlm_to_host(out, 2, p->stream);
 }
 
 void fill_common(nlm_plan* p, KParams& kp) {
@@ -920,9 +920,8 @@ extern "C" int nlm_batch_grids(nlm_plan* p, const double* inputs, int rows, int 
   tic(p, 2);
   if (int e = launch_prop_kernel(p, kp)) return e;
   tic(p, 3);
-  if (grid_freq) HIP_TRY(hipMemcpyAsync(grid_freq, p->gridF.p, g * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (grid_time) HIP_TRY(hipMemcpyAsync(grid_time, p->gridT.p, g * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  const HostCopy out[2] = {{grid_freq, p->gridF.p, g * sizeof(cplx)}, {grid_time, p->gridT.p, g * sizeof(cplx)}};
+  if (int e = nlm_to_host(out, 2, p->stream)) return e;
   if (p->timing) collect_timing(p, 2, 3, 1);
   return NLM_OK;
 }
@@ -932,10 +931,8 @@ extern "C" int nlm_grid_download(nlm_plan* p, int mode, double* sf, double* st) 
   if (mode < 0 || mode >= p->nS) return set_err(NLM_INVALID_ARGUMENT, "mode index out of range");
   if (!p->gridF.p) return set_err(NLM_RUNTIME_ERROR, "no signal grid has been computed");
   const size_t cnt = (size_t)p->nZ * p->N, off = (size_t)mode * cnt;
-  if (sf) HIP_TRY(hipMemcpyAsync(sf, p->gridF.p + off, cnt * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (st) HIP_TRY(hipMemcpyAsync(st, p->gridT.p + off, cnt * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
-  return NLM_OK;
+  const HostCopy out[2] = {{sf, p->gridF.p + off, cnt * sizeof(cplx)}, {st, p->gridT.p + off, cnt * sizeof(cplx)}};
+  return nlm_to_host(out, 2, p->stream);
 }
 
 static int batch_common(nlm_plan* p, const cplx* in_dev, int rows, int cols, int in_time, int input_mode, int n_out,
@@ -985,10 +982,8 @@ extern "C" int nlm_batch(nlm_plan* p, const double* inputs, int rows, int cols, 
   if (int e = upload(p->in, inputs, (size_t)rows * cols, p->stream)) return e;
   if (int e = p->out.ensure((size_t)rows * n_out * p->N)) return e;
   if (int e = batch_common(p, p->in.p, rows, cols, in_time, input_mode, n_out, outputs, p->out.p)) return e;
-  if (out && rows > 0)
-    HIP_TRY(hipMemcpyAsync(out, p->out.p, (size_t)rows * n_out * p->N * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
-  return NLM_OK;
+  const HostCopy res = {out, p->out.p, (size_t)rows * n_out * p->N * sizeof(cplx)};
+  return nlm_to_host(&res, 1, p->stream);
 }
 
 extern "C" int nlm_batch_dev(nlm_plan* p, const double* in_dev, int rows, int cols, int in_time, int input_mode,
@@ -1046,9 +1041,8 @@ extern "C" int nlm_greens(nlm_plan* p, int in_time, int n_in, const int32_t* inp
   tic(p, 4);
   p->greensRows = (int)W;
   p->greensCols = n_in * N;
-  if (C) HIP_TRY(hipMemcpyAsync(C, p->C.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (S) HIP_TRY(hipMemcpyAsync(S, p->S.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
+  const HostCopy out[2] = {{C, p->C.p, total * sizeof(cplx)}, {S, p->S.p, total * sizeof(cplx)}};
+  if (int e = nlm_to_host(out, 2, p->stream)) return e;
   scale.release();
   if (p->timing) {
     collect_timing(p, 2, 3, 1);
@@ -1061,10 +1055,8 @@ extern "C" int nlm_greens_download(nlm_plan* p, double* C, double* S) {
   if (!p) return set_err(NLM_INVALID_ARGUMENT, "null plan");
   if (!p->greensRows) return set_err(NLM_RUNTIME_ERROR, "no Green's function has been computed");
   const size_t total = (size_t)p->greensRows * p->greensCols;
-  if (C) HIP_TRY(hipMemcpyAsync(C, p->C.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  if (S) HIP_TRY(hipMemcpyAsync(S, p->S.p, total * sizeof(cplx), hipMemcpyDeviceToHost, p->stream));
-  HIP_TRY(hipStreamSynchronize(p->stream));
-  return NLM_OK;
+  const HostCopy out[2] = {{C, p->C.p, total * sizeof(cplx)}, {S, p->S.p, total * sizeof(cplx)}};
+  return nlm_to_host(out, 2, p->stream);
 }
 
 int nlm_fft_device(const cplx* in, cplx* out, int n, int count, bool inverse, hipStream_t s) {

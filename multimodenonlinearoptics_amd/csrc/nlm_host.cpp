@@ -175,15 +175,22 @@ void Medium::resetGrids(unsigned nFreqs, double tMax) {
   signalTime_.assign(nS_, Grid());
 }
 
-void Medium::allocPump(unsigned q) {
-  if (pumpFreq_[q].rows != nZP_ || pumpFreq_[q].cols != N_) pumpFreq_[q].setZero(nZP_, N_);
-  if (pumpTime_[q].rows != nZP_ || pumpTime_[q].cols != N_) pumpTime_[q].setZero(nZP_, N_);
+// `written`: a download fills the grid next, so a new one need not be zeroed first
+static void allocGrid(Grid& g, int rows, int cols, bool written) {
+  if (g.rows == rows && g.cols == cols) return;
+  if (written) g.setSize(rows, cols);
+  else g.setZero(rows, cols);
 }
 
-void Medium::allocSignal() {
+void Medium::allocPump(unsigned q, bool written) {
+  allocGrid(pumpFreq_[q], nZP_, N_, written);
+  allocGrid(pumpTime_[q], nZP_, N_, written);
+}
+
+void Medium::allocSignal(bool written) {
   for (int m = 0; m < nS_; m++) {
-    if (signalFreq_[m].rows != nZ_ || signalFreq_[m].cols != N_) signalFreq_[m].setZero(nZ_, N_);
-    if (signalTime_[m].rows != nZ_ || signalTime_[m].cols != N_) signalTime_[m].setZero(nZ_, N_);
+    allocGrid(signalFreq_[m], nZ_, N_, written);
+    allocGrid(signalTime_[m], nZ_, N_, written);
   }
 }
 
@@ -425,8 +432,9 @@ void Medium::markPumpOnDevice() {
 }
 
 void Medium::syncPumpToHost(unsigned i) {
-  if ((int)i < nP_) allocPump(i);
-  if (i < pumpHostStale_.size() && pumpHostStale_[i] && plan_) {
+  const bool stale = i < pumpHostStale_.size() && pumpHostStale_[i] && plan_;
+  if ((int)i < nP_) allocPump(i, stale);
+  if (stale) {
     check(nlm_pump_download(plan_, (int)i, reinterpret_cast<double*>(pumpTime_[i].v.data()),
                             reinterpret_cast<double*>(pumpFreq_[i].v.data())));
     pumpHostStale_[i] = false;
@@ -434,8 +442,9 @@ void Medium::syncPumpToHost(unsigned i) {
 }
 
 void Medium::syncSignalToHost() {
-  allocSignal();
-  if (signalHostStale_ && plan_) {
+  const bool stale = signalHostStale_ && plan_;
+  allocSignal(stale);
+  if (stale) {
     for (int m = 0; m < nS_; m++)
       check(nlm_grid_download(plan_, m, reinterpret_cast<double*>(signalFreq_[m].v.data()),
                               reinterpret_cast<double*>(signalTime_[m].v.data())));
@@ -530,8 +539,8 @@ std::pair<Grid, Grid> Medium::batchSignalGrids(const Grid& in, bool inTimeDomain
     pumpComputed_ = true;
   }
   std::pair<Grid, Grid> g;
-  g.first.setZero(in.rows * nS_ * nZ_, N_);
-  g.second.setZero(in.rows * nS_ * nZ_, N_);
+  g.first.setSize(in.rows * nS_ * nZ_, N_);
+  g.second.setSize(in.rows * nS_ * nZ_, N_);
   check(nlm_batch_grids(p, reinterpret_cast<const double*>(in.v.data()), in.rows, in.cols, inTimeDomain ? 1 : 0,
                         (int)inputMode, reinterpret_cast<double*>(g.first.v.data()),
                         reinterpret_cast<double*>(g.second.v.data())));
@@ -572,24 +581,41 @@ void Medium::greensOnDevice(bool inTimeDomain, bool runPump) {
   greensImpl(inTimeDomain, runPump, 1, false, {}, {}, false);
 }
 
-std::pair<Grid, Grid> Medium::greensForward(bool inTimeDomain, bool runPump, int ckptEvery) {
+void Medium::greensForwardReady(bool runPump) {
   if (model_ != NLM_CHI2PDC) throw std::invalid_argument("the differentiable Green's function is implemented for Chi2PDC");
   if (runPump) runPumpSimulation();
-  nlm_plan* p = plan();
+  plan();
   for (int q = 0; q < nP_; q++)
     if (pumpDevStale_[q]) uploadPump(q);
   if (nP_ > 0 && !pumpComputed_) {
     for (int q = 0; q < nP_; q++) uploadPump(q);
     pumpComputed_ = true;
   }
+}
+
+std::pair<Grid, Grid> Medium::greensForward(bool inTimeDomain, bool runPump, int ckptEvery) {
+  greensForwardReady(runPump);
   std::pair<Grid, Grid> res;
-  res.first.setZero(N_, N_);
-  res.second.setZero(N_, N_);
+  res.first.setSize(N_, N_);
+  res.second.setSize(N_, N_);
   const int32_t m0 = 0;
-  check(nlm_greens_forward(p, inTimeDomain ? 1 : 0, 1, &m0, 1, &m0, nullptr, ckptEvery,
+  check(nlm_greens_forward(plan(), inTimeDomain ? 1 : 0, 1, &m0, 1, &m0, nullptr, ckptEvery,
                            reinterpret_cast<double*>(res.first.v.data()), reinterpret_cast<double*>(res.second.v.data())));
   ++forwardSerial_;
   return res;
+}
+
+bool Medium::onDevice(const std::vector<std::uintptr_t>& ptrs) {
+  for (std::uintptr_t q : ptrs)
+    if (!nlm_plan_owns_device_of(plan(), reinterpret_cast<const void*>(q))) return false;
+  return true;
+}
+
+void Medium::greensForwardDev(bool inTimeDomain, bool runPump, int ckptEvery, std::uintptr_t C, std::uintptr_t S) {
+  greensForwardReady(runPump);
+  check(nlm_greens_forward_dev(plan(), inTimeDomain ? 1 : 0, ckptEvery, reinterpret_cast<double*>(C),
+                               reinterpret_cast<double*>(S)));
+  ++forwardSerial_;
 }
 
 // Chain rule from the step coefficients to the per-step poling values for
@@ -599,10 +625,21 @@ std::pair<std::vector<cd>, std::vector<double>> Medium::greensAdjoint(const cd* 
                                                                       int cols) {
   if (model_ != NLM_CHI2PDC) throw std::invalid_argument("the differentiable Green's function is implemented for Chi2PDC");
   if (rows != N_ || cols != N_) throw std::invalid_argument("gradient shapes do not match the Green's function");
-  nlm_plan* p = plan();
   std::vector<cd> gcoef((size_t)nZ_ * 3), genv(N_);
-  check(nlm_greens_adjoint(p, reinterpret_cast<const double*>(gC), reinterpret_cast<const double*>(gS),
+  check(nlm_greens_adjoint(plan(), reinterpret_cast<const double*>(gC), reinterpret_cast<const double*>(gS),
                            reinterpret_cast<double*>(gcoef.data()), nullptr, reinterpret_cast<double*>(genv.data())));
+  return {genv, polingGradient(gcoef)};
+}
+
+std::pair<std::vector<cd>, std::vector<double>> Medium::greensAdjointDev(std::uintptr_t gC, std::uintptr_t gS) {
+  if (model_ != NLM_CHI2PDC) throw std::invalid_argument("the differentiable Green's function is implemented for Chi2PDC");
+  std::vector<cd> gcoef((size_t)nZ_ * 3), genv(N_);
+  check(nlm_greens_adjoint_dev(plan(), reinterpret_cast<const double*>(gC), reinterpret_cast<const double*>(gS),
+                               reinterpret_cast<double*>(gcoef.data()), reinterpret_cast<double*>(genv.data())));
+  return {genv, polingGradient(gcoef)};
+}
+
+std::vector<double> Medium::polingGradient(const std::vector<cd>& gcoef) const {
   std::vector<double> gpol(nZ_, 0.0);
   for (unsigned i = 1; i < (unsigned)nZ_; i++) {
     const double x[3] = {(i - 1) * dz_, (i - .5) * dz_, i * dz_};
@@ -612,7 +649,7 @@ std::pair<std::vector<cd>, std::vector<double>> Medium::greensAdjoint(const cd* 
     gpol[i - 1] += a0 + 0.5 * a1;
     gpol[i] += 0.5 * a1 + a2;
   }
-  return {genv, gpol};
+  return gpol;
 }
 
 // Differentiable batchSignalSimulation of a fully nonlinear medium
@@ -622,7 +659,7 @@ Grid Medium::batchForward(const Grid& in, bool inTimeDomain, int ckptEvery) {
   if (in.cols != N_) throw std::invalid_argument("Signals not of correct length!");
   if (in.rows == 0) throw std::invalid_argument("empty batch");
   Grid out;
-  out.setZero(in.rows, N_);
+  out.setSize(in.rows, N_);
   check(nlm_batch_forward(plan(), reinterpret_cast<const double*>(in.v.data()), in.rows, inTimeDomain ? 1 : 0,
                           ckptEvery, reinterpret_cast<double*>(out.v.data())));
   batchRows_ = in.rows;
@@ -636,9 +673,24 @@ Grid Medium::batchAdjoint(const Grid& gOut) {
   if (gOut.rows != batchRows_ || gOut.cols != N_)
     throw std::invalid_argument("gradient shape does not match the last batchForward");
   Grid g;
-  g.setZero(gOut.rows, N_);
+  g.setSize(gOut.rows, N_);
   check(nlm_batch_adjoint(plan(), reinterpret_cast<const double*>(gOut.v.data()), reinterpret_cast<double*>(g.v.data())));
   return g;
+}
+
+void Medium::batchForwardDev(std::uintptr_t in, int rows, bool inTimeDomain, int ckptEvery, std::uintptr_t out) {
+  if (model_ != NLM_CHI3GNLSE) throw std::invalid_argument("the differentiable batch is implemented for Chi3GNLSE");
+  if (rows == 0) throw std::invalid_argument("empty batch");
+  check(nlm_batch_forward_dev(plan(), reinterpret_cast<const double*>(in), rows, inTimeDomain ? 1 : 0, ckptEvery,
+                              reinterpret_cast<double*>(out)));
+  batchRows_ = rows;
+  ++forwardSerial_;
+}
+
+void Medium::batchAdjointDev(std::uintptr_t gOut, std::uintptr_t gIn) {
+  if (model_ != NLM_CHI3GNLSE) throw std::invalid_argument("the differentiable batch is implemented for Chi3GNLSE");
+  if (batchRows_ == 0) throw std::runtime_error("run batchForward before batchAdjoint");
+  check(nlm_batch_adjoint_dev(plan(), reinterpret_cast<const double*>(gOut), reinterpret_cast<double*>(gIn)));
 }
 
 void Medium::enableTiming(bool on) { check(nlm_plan_enable_timing(plan(), on ? 1 : 0)); }
@@ -689,8 +741,8 @@ std::pair<Grid, Grid> Medium::greensImpl(bool inTimeDomain, bool runPump, unsign
   lastGreensRows_ = nOut * N_;
   lastGreensCols_ = nIn * N_;
   if (download) {
-    res.first.setZero(nOut * N_, nIn * N_);
-    res.second.setZero(nOut * N_, nIn * N_);
+    res.first.setSize(nOut * N_, nIn * N_);
+    res.second.setSize(nOut * N_, nIn * N_);
   }
   check(nlm_greens(p, inTimeDomain ? 1 : 0, nIn, ins.data(), nOut, outs.data(),
                    normalize ? reinterpret_cast<const double*>(scale.data()) : nullptr,
@@ -726,7 +778,7 @@ Grid Medium::batchSignalSimulation(const Grid& in, bool inTimeDomain, bool runPu
     pumpComputed_ = true;
   }
   Grid out;
-  out.setZero(nInputs, nOut * N_);
+  out.setSize(nInputs, nOut * N_);
   check(nlm_batch(p, reinterpret_cast<const double*>(in.v.data()), nInputs, inCols, inTimeDomain ? 1 : 0,
                   (int)inputMode, nOut, outs.data(), reinterpret_cast<double*>(out.v.data())));
   return out;
@@ -1318,8 +1370,8 @@ std::pair<Grid, Grid> Cascade::computeGreensFunction(bool inTimeDomain, bool run
     if (last) rows = m.lastGreensRows_;
   }
   std::pair<Grid, Grid> res;
-  res.first.setZero(rows, cols);
-  res.second.setZero(rows, cols);
+  res.first.setSize(rows, cols);
+  res.second.setSize(rows, cols);
   check(nlm_greens_cascade((int)plans.size(), plans.data(), reinterpret_cast<double*>(res.first.v.data()),
                            reinterpret_cast<double*>(res.second.v.data())));
   return res;

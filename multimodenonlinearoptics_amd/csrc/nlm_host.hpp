@@ -10,12 +10,16 @@
 #pragma once
 #include <complex>
 #include <cstdint>
+#include <sys/mman.h>
+
 #include <array>
 #include <map>
 #include <memory>
 #include <stdexcept>
 #include <string>
 #include <utility>
+#include <cstdlib>
+#include <new>
 #include <vector>
 
 #include "nlm.h"
@@ -28,13 +32,51 @@ enum class PulseType : int { Gaussian = 0, Sech = 1, Sinc = 2 };
 enum class IntensityProfile : int { GaussianBeam = 0, Constant = 1, GaussianApodization = 2 };
 
 // Row-major 2-D complex array (the reference's Array2Dcd).
+// Memory of a host array: elements are left unset until written (results are filled
+// by the device), and arrays of 2 MB and more lie on huge pages where the system
+// offers them, which cost one page fault instead of 512 when they are first filled.
+template <class T>
+struct ArrayAllocator {
+  using value_type = T;
+  ArrayAllocator() = default;
+  template <class U>
+  ArrayAllocator(const ArrayAllocator<U>&) {}
+  T* allocate(size_t n) {
+    constexpr size_t huge = (size_t)2 << 20;
+    const size_t bytes = n * sizeof(T);
+    void* p = nullptr;
+    if (bytes >= huge) {
+      if (posix_memalign(&p, huge, bytes)) throw std::bad_alloc();
+      (void)madvise(p, bytes / huge * huge, MADV_HUGEPAGE);
+    } else if (!(p = std::malloc(bytes ? bytes : 1))) {
+      throw std::bad_alloc();
+    }
+    return static_cast<T*>(p);
+  }
+  void deallocate(T* p, size_t) { std::free(p); }
+  template <class U>
+  void construct(U*) {}
+  template <class U, class... A>
+  void construct(U* p, A&&... a) {
+    ::new ((void*)p) U(std::forward<A>(a)...);
+  }
+  bool operator==(const ArrayAllocator&) const { return true; }
+  bool operator!=(const ArrayAllocator&) const { return false; }
+};
+
 struct Grid {
   int rows = 0, cols = 0;
-  std::vector<cd> v;
+  std::vector<cd, ArrayAllocator<cd>> v;
   void setZero(int r, int c) {
     rows = r;
     cols = c;
     v.assign((size_t)r * c, cd(0, 0));
+  }
+  // r x c elements with unset values, for a result that is then written whole
+  void setSize(int r, int c) {
+    rows = r;
+    cols = c;
+    v.resize((size_t)r * c);
   }
   cd* row(int i) { return v.data() + (size_t)i * cols; }
   const cd* row(int i) const { return v.data() + (size_t)i * cols; }
@@ -109,6 +151,15 @@ class Medium {
   // shape (rows * nS * nZ, N), frequency and time domain
   std::pair<Grid, Grid> batchSignalGrids(const Grid& inputProfs, bool inTimeDomain, unsigned inputMode);
   Grid batchAdjoint(const Grid& gOut);
+  // The same on arrays in device memory of the plan's device (addresses); false where
+  // the engine's HIP runtime does not know them as such, before anything has run.
+  bool onDevice(const std::vector<std::uintptr_t>& ptrs);
+  void greensForwardReady(bool runPump);
+  std::vector<double> polingGradient(const std::vector<cd>& gcoef) const;
+  void greensForwardDev(bool inTimeDomain, bool runPump, int ckptEvery, std::uintptr_t C, std::uintptr_t S);
+  std::pair<std::vector<cd>, std::vector<double>> greensAdjointDev(std::uintptr_t gC, std::uintptr_t gS);
+  void batchForwardDev(std::uintptr_t in, int rows, bool inTimeDomain, int ckptEvery, std::uintptr_t out);
+  void batchAdjointDev(std::uintptr_t gOut, std::uintptr_t gIn);
   void enableTiming(bool on);
   void setStepTable(bool on);
   std::vector<double> lastTiming();
@@ -177,8 +228,8 @@ class Medium {
   std::vector<std::vector<double>> dispPump_, dispSign_;
   std::vector<std::vector<cd>> dispStepPump_, dispStepSign_;
   std::vector<Grid> pumpFreq_, pumpTime_, signalFreq_, signalTime_, field_;
-  void allocPump(unsigned q);
-  void allocSignal();
+  void allocPump(unsigned q, bool written = false);
+  void allocSignal(bool written = false);
   std::vector<cd> raman_;
 
   nlm_plan* plan_ = nullptr;

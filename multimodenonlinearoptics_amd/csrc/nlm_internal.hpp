@@ -46,6 +46,19 @@ struct DevBuf {
   }
 };
 
+// Copies to and from a caller's pageable memory (nlm_copy.hip).  nlm_to_host returns
+// when every item is in place (items with a null host pointer are skipped) and the
+// stream's work before it is done; nlm_to_device when `host` may be reused.
+struct HostCopy {
+  void* host;
+  const void* dev;
+  size_t bytes;
+};
+int nlm_to_host(const HostCopy* items, int n, hipStream_t s);
+int nlm_to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
+// whether ptr is memory of `device` that this process's HIP runtime knows
+bool nlm_on_device(const void* ptr, int device);
+
 struct nlm_plan_s {
   int model = 0, N = 0, L = 0, nZ = 0, nS = 0, nP = 0, NC = 0, NCC = 0;
   int device = 0;
@@ -65,6 +78,7 @@ struct nlm_plan_s {
   double dzp = 0;
   DevBuf<cplx> ckpt, gG, gC, gS, gcoefPart, gcoef, gpumpPart, gpump, gF0Part, gF0, gtmp, gslice;
   DevBuf<cplx> scale;
+  DevBuf<cplx> cascade[2][2];  // products of nlm_greens_cascade whose last plan this is
   // staged transform for Chi3GNLSE with nFreqs > 8192 (nlm_big.hip)
   DevBuf<cplx> bigState, bigH;
   DevBuf<int> bigBase;

@@ -263,6 +263,44 @@ PYBIND11_MODULE(nonlinearmedium, m) {
            },
            "Gradients (dL/d envelope, dL/d poling profile) of the last greensForward for dL/dC, dL/dS "
            "(convention dL/dRe + i dL/dIm) (extension; Chi2PDC).", "gC"_a, "gS"_a);
+  // The same on device memory: addresses (tensor.data_ptr()) of contiguous complex128
+  // matrices of the medium's device, whose pending work is complete.
+  base.def("onDevice", [](Medium& md, const std::vector<std::uintptr_t>& ptrs) { return md.onDevice(ptrs); },
+           "Whether every address is memory of the medium's device known to the engine (extension).", "ptrs"_a);
+  base.def("greensForwardDev",
+           [](Medium& md, std::uintptr_t C, std::uintptr_t S, bool inTimeDomain, bool runPump, int ckptEvery) {
+             py::gil_scoped_release nogil;
+             md.greensForwardDev(inTimeDomain, runPump, ckptEvery, C, S);
+           },
+           "greensForward into device matrices (extension; Chi2PDC).", "C"_a, "S"_a, "inTimeDomain"_a = false,
+           "runPump"_a = true, "ckptEvery"_a = 0);
+  base.def("greensAdjointDev",
+           [](Medium& md, std::uintptr_t gC, std::uintptr_t gS) {
+             std::pair<std::vector<cd>, std::vector<double>> r;
+             {
+               py::gil_scoped_release nogil;
+               r = md.greensAdjointDev(gC, gS);
+             }
+             py::array_t<std::complex<double>> ge(r.first.size());
+             std::copy(r.first.begin(), r.first.end(), ge.mutable_data());
+             py::array_t<double> gp(r.second.size());
+             std::copy(r.second.begin(), r.second.end(), gp.mutable_data());
+             return py::make_tuple(ge, gp);
+           },
+           "greensAdjoint of device matrices (extension; Chi2PDC).", "gC"_a, "gS"_a);
+  base.def("batchForwardDev",
+           [](Medium& md, std::uintptr_t in, int rows, std::uintptr_t out, bool inTimeDomain, int ckptEvery) {
+             py::gil_scoped_release nogil;
+             md.batchForwardDev(in, rows, inTimeDomain, ckptEvery, out);
+           },
+           "batchForward of a device matrix [rows, nFreqs] into another (extension; Chi3GNLSE).", "inputs"_a, "rows"_a,
+           "out"_a, "inTimeDomain"_a = true, "ckptEvery"_a = 0);
+  base.def("batchAdjointDev",
+           [](Medium& md, std::uintptr_t gOut, std::uintptr_t gIn) {
+             py::gil_scoped_release nogil;
+             md.batchAdjointDev(gOut, gIn);
+           },
+           "batchAdjoint of a device matrix into another (extension; Chi3GNLSE).", "gOut"_a, "gIn"_a);
   base.def("batchSignalGrids",
            [](Medium& md, const carr& in, bool inTimeDomain, unsigned inputMode) {
              Grid g = to_grid(in);
