@@ -150,7 +150,8 @@ __global__ void __launch_bounds__(Launch<L>::THREADS)
   store_row<L>(pumpT + (size_t)i * N, f, t, active && !lastRow);
 }
 
-// Chi3 nonlinear pump, serial over 2nZ-1 rows (solvers/Chi3.cpp:25-54).
+// Chi3 nonlinear pump, serial over 2nZ-1 rows (solvers/Chi3.cpp:25-54): one field, so the
+// time is one wave's chain of two transforms and a phase per row.
 template <int L>
 __global__ void __launch_bounds__(FftShape<L>::T) k_pump_chi3(const cplx* __restrict__ env, const double* __restrict__ Dp,
                                                               double dzp, const cplx* __restrict__ dstepP,
@@ -159,17 +160,18 @@ __global__ void __launch_bounds__(FftShape<L>::T) k_pump_chi3(const cplx* __rest
                                                               const cplx* __restrict__ twt) {
   using F = FftShape<L>;
   constexpr int N = F::N, T = F::T;
+  constexpr bool WAVE = T <= 64;  // the workgroup is one wave
   __shared__ cplx buf[F::lds_elems];
   const int t = threadIdx.x;
-  FftTwiddles<L> tw;
-  fft_load_twiddles<L>(tw, twt, t);
+  RegTwiddles<L> tw;
+  fft_load_twiddles<L>(tw.w, twt, t);
   cplx v[8], dsp[8];
 #pragma unroll
   for (int m = 0; m < 8; m++) {
     v[m] = env[t + T * m];
     dsp[m] = dstepP[t + T * m];
   }
-  fft_field<L, false>(v, buf, t, tw);
+  fft_field1<L, false, WAVE>(v, buf, t, tw);
 #pragma unroll
   for (int m = 0; m < 8; m++) {
     double s, c;
@@ -177,20 +179,15 @@ __global__ void __launch_bounds__(FftShape<L>::T) k_pump_chi3(const cplx* __rest
     v[m] = v[m] * mk(c, s);
   }
   store_row<L>(pumpF, v, t, true);
-  fft_field<L, true>(v, buf, t, tw);
+  fft_field1<L, true, WAVE>(v, buf, t, tw);
   scale_inv<L>(v);
   store_row<L>(pumpT, v, t, true);
+  cplx next = relI[0];
   for (int i = 1; i < nZP; i++) {
-    const cplx r = relI[i - 1];
-#pragma unroll
-    for (int m = 0; m < 8; m++) {
-      const double a2 = abs2(v[m]);
-      const double e = exp(r.re * a2);
-      double s, c;
-      sincos(r.im * a2, &s, &c);
-      v[m] = v[m] * mk(e * c, e * s);
-    }
-    fft_field<L, false>(v, buf, t, tw);
+    const cplx r = next;
+    next = relI[i];  // nZP entries; the last is not used
+    self_phase<8>(v, r);
+    fft_field1<L, false, WAVE>(v, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) v[m] = v[m] * dsp[m];
     if (i == nZP - 1) {
@@ -202,7 +199,7 @@ __global__ void __launch_bounds__(FftShape<L>::T) k_pump_chi3(const cplx* __rest
       }
     }
     store_row<L>(pumpF + (size_t)i * N, v, t, true);
-    fft_field<L, true>(v, buf, t, tw);
+    fft_field1<L, true, WAVE>(v, buf, t, tw);
     scale_inv<L>(v);
     store_row<L>(pumpT + (size_t)i * N, v, t, true);
   }

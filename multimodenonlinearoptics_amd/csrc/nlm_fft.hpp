@@ -109,6 +109,62 @@ __device__ __forceinline__ void sincos_reduced(double a, double* s, double* c) {
   }
 }
 
+// sin and cos for |x| <= pi/4, without a branch, so that the points of a lane overlap.
+// With z = x^2: sin x = x + x z S(z), cos x = (1 - z/2) + (z^2 C(z) + the rounding error
+// of 1 - z/2).  S (degree 6) and C (degree 5) interpolate the exact series at the Chebyshev
+// nodes of [0, (pi/4)^2]; truncation below 1e-18, results within 0.55 ulp like the library's.
+__device__ __forceinline__ void sincos_small(double x, double* s, double* c) {
+  const double z = x * x;
+  double p = -7.586691094197958e-13;
+  p = fma(p, z, 1.6058531516797758e-10);
+  p = fma(p, z, -2.5052106231802837e-08);
+  p = fma(p, z, 2.7557319219337312e-06);
+  p = fma(p, z, -0.00019841269841265063);
+  p = fma(p, z, 0.008333333333333331);
+  p = fma(p, z, -0.16666666666666666);
+  *s = fma(x * z, p, x);
+  double q = -1.1382623647474604e-11;
+  q = fma(q, z, 2.087614614655861e-09);
+  q = fma(q, z, -2.7557317271145144e-07);
+  q = fma(q, z, 2.480158729876456e-05);
+  q = fma(q, z, -0.0013888888888887398);
+  q = fma(q, z, 0.041666666666666664);
+  const double h = fma(-0.5, z, 1.0);
+  *c = h + fma(z * z, q, fma(-0.5, z, 1.0 - h));
+}
+
+// v *= exp(q |v|^2): a step of the self-phase modulated pump.  q is purely imaginary for a
+// lossless medium: exp(0) is exactly 1 and is left out, and a resolved step turns the phase
+// by far less than pi/4; both tests are the same for all lanes of a wave, any other wave
+// takes the library's exp and sincos.  8 points per lane, N = 512, 1999 rows: 6.7 -> 4.5 ms
+// for the whole pump together with the wave-local exchanges.
+template <int R>
+__device__ __forceinline__ void self_phase(cplx* v, cplx q) {
+  double a[R], top = 0;
+#pragma unroll
+  for (int m = 0; m < R; m++) {
+    a[m] = abs2(v[m]);
+    top = fmax(top, fabs(q.im * a[m]));
+    if (!(a[m] <= 1.7976931348623157e308)) top = 1e300;  // infinite or NaN
+  }
+  if (q.re == 0.0 && __all(top <= 0.78539816339744828)) {
+#pragma unroll
+    for (int m = 0; m < R; m++) {
+      double s, c;
+      sincos_small(q.im * a[m], &s, &c);
+      v[m] = v[m] * mk(c, s);
+    }
+    return;
+  }
+#pragma unroll
+  for (int m = 0; m < R; m++) {
+    const double e = exp(q.re * a[m]);
+    double s, c;
+    sincos(q.im * a[m], &s, &c);
+    v[m] = v[m] * mk(e * c, e * s);
+  }
+}
+
 // Workgroup barrier ordering LDS only: unlike __syncthreads() it does not wait
 // for outstanding global loads, so loads issued before a transform (the next
 // z step's pump rows) stay in flight across its LDS exchanges.

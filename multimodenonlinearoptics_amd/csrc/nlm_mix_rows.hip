@@ -80,14 +80,7 @@ __global__ void __launch_bounds__(MIX_MAX_THREADS) k_mix_pump_chi3(MixRows r, Mi
   mix::put_row(f, r.pumpT, v, act);
   for (int i = 1; i < r.nZP; i++) {
     const cplx q = r.relI[i - 1];
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const double a2 = abs2(v[k]);
-      const double e = exp(q.re * a2);
-      double s, c;
-      sincos(q.im * a2, &s, &c);
-      v[k] = v[k] * mk(e * c, e * s);
-    }
+    self_phase<R>(v, q);
     f.template run<false>(v);
 #pragma unroll
     for (int k = 0; k < R; k++) v[k] = v[k] * dsp[k];
