@@ -451,64 +451,61 @@ __device__ __forceinline__ void table_field(const KParams& kp, Fft<R>& f, int fi
   leave<1>(kp, f, field, 0, act, v);
 }
 
-// k = IFFT( FFT( IFFT(FFT(r |y|^2) * R) * y ) * (nl0 + nl1*omega) ), solvers/Chi3GNLSE.cpp:51-92
-template <int R>
-__device__ __forceinline__ void gnlse_stage(const KParams& kp, Fft<R>& f, const cplx (&y)[R], double r, cplx (&k)[R]) {
-#pragma unroll
-  for (int m = 0; m < R; m++) k[m] = mk(r * abs2(y[m]), 0.0);
-  f.template run<false>(k);
-  mul_row(f, k, kp.raman);
-  f.template run<true>(k);
-  scale_row(f, k);
-#pragma unroll
-  for (int m = 0; m < R; m++) k[m] = k[m] * y[m];
-  f.template run<false>(k);
-  mul_row(f, k, kp.filt);
-  f.template run<true>(k);
-  scale_row(f, k);
-}
-
+// One Chi3GNLSE field (solvers/Chi3GNLSE.cpp:51-92), state and RK4 sum kept as spectra as in
+// the power-of-two kernel (16 transforms per step): FFT(k) of a stage is
+// filter FFT( IFFT(FFT(r |y|^2) R) y ).
 template <int R>
 __device__ __forceinline__ void gnlse_field(const KParams& kp, Fft<R>& f, int field, bool act) {
   const int N = f.p.N;
-  cplx v[R];
+  cplx v[R], y[R];  // v: spectrum; y: time-domain stage input
   enter<1>(kp, f, field, 0, act, v);
   if (kp.nZ > 1) {
-    f.template run<true>(v);
-    scale_row(f, v);
-    if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), v, act);
+#pragma unroll
+    for (int m = 0; m < R; m++) y[m] = v[m];
+    f.template run<true>(y);
+    scale_row(f, y);
+    if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, 0, N), y, act);
   }
   for (int i = 1; i < kp.nZ; i++) {
     const uniform_cplx* c = to_uniform(kp.coef + (size_t)i * 3);
     // acc accumulates ((k1 + 2 k2) + 2 k3) + k4 in the reference's order
-    cplx y[R], k[R], acc[R];
+    cplx acc[R];
 #pragma unroll
-    for (int m = 0; m < R; m++) {
-      y[m] = v[m];
-      acc[m] = mk(0.0, 0.0);
-    }
+    for (int m = 0; m < R; m++) acc[m] = mk(0.0, 0.0);
     // one copy of the four transforms for the four stages
 #pragma unroll 1
     for (int s = 0; s < 4; s++) {
       const double r = s == 0 ? c[0].re : s == 3 ? c[2].re : c[1].re;
-      gnlse_stage<R>(kp, f, y, r, k);
+      cplx k[R];
+#pragma unroll
+      for (int m = 0; m < R; m++) k[m] = mk(r * abs2(y[m]), 0.0);
+      f.template run<false>(k);
+      mul_row(f, k, kp.raman);
+      f.template run<true>(k);
+      scale_row(f, k);
+#pragma unroll
+      for (int m = 0; m < R; m++) k[m] = k[m] * y[m];
+      f.template run<false>(k);
+      mul_row(f, k, kp.filt);
       const double wa = s == 1 || s == 2 ? 2.0 : 1.0, wy = s == 2 ? 1.0 : 0.5;
 #pragma unroll
-      for (int m = 0; m < R; m++) {
-        acc[m] = acc[m] + wa * k[m];
-        y[m] = v[m] + wy * k[m];
-      }
-    }
+      for (int m = 0; m < R; m++) acc[m] = acc[m] + wa * k[m];
+      if (s < 3) {
 #pragma unroll
-    for (int m = 0; m < R; m++) v[m] = v[m] + acc[m] * (1. / 6.);
-    f.template run<false>(v);
-    mul_row(f, v, kp.dstep);
-    if (i < kp.nZ - 1) {
-      if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
-      f.template run<true>(v);
-      scale_row(f, v);
-      if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), v, act);
+        for (int m = 0; m < R; m++) y[m] = v[m] + wy * k[m];
+      } else {
+#pragma unroll
+        for (int m = 0; m < R; m++) v[m] = v[m] + acc[m] * (1. / 6.);
+        mul_row(f, v, kp.dstep);
+        if (i == kp.nZ - 1) break;
+        if (kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridF, field, 1, 0, i, N), v, act);
+#pragma unroll
+        for (int m = 0; m < R; m++) y[m] = v[m];
+      }
+      f.template run<true>(y);
+      scale_row(f, y);
     }
+    if (i < kp.nZ - 1 && kp.kind == KIND_GRID) put_row(f, grid_row(kp, kp.gridT, field, 1, 0, i, N), y, act);
   }
   leave<1>(kp, f, field, 0, act, v);
 }

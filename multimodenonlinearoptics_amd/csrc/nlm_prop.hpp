@@ -420,90 +420,128 @@ __global__ void __launch_bounds__(Launch<L>::THREADS) k_prop(KParams kp) {
   prop_field<M, L>(kp, field, field < kp.nFields, t, lds + lf * F::lds_elems, twl);
 }
 
+template <int L>
+__device__ __forceinline__ void store_scaled(cplx* __restrict__ dst, const cplx (&v)[8], int t, bool active) {
+  constexpr int T = FftShape<L>::T;
+  constexpr double s = 1.0 / FftShape<L>::N;
+  if (active) {
+#pragma unroll
+    for (int m = 0; m < 8; m++) dst[t + T * m] = v[m] * s;
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Chi3GNLSE: transforms inside every RK stage (solvers/Chi3GNLSE.cpp:51-92)
 // ---------------------------------------------------------------------------
 
-// k = IFFT( FFT( IFFT(FFT(r |y|^2) * R) * y ) * (nl0 + nl1*omega) )
-template <int L, class TW>
-__device__ __forceinline__ void gnlse_stage(const cplx (&y)[8], double r, cplx (&k)[8], const cplx (&ram)[8],
-                                            const cplx (&flt)[8], cplx* buf, int t, const TW& tw) {
+// A spectral row of the GNLSE step: held in registers, or (MEM, from N = 4096, where a lane
+// has 256 or 128) fetched before the last exchange of the transform in front of its use.
+template <int L, bool MEM>
+struct SpectralRow {
+  cplx h[MEM ? 1 : 8];
+  const cplx* src;
+  __device__ __forceinline__ void init(const cplx* row, int t) {
+    src = row;
+    if constexpr (!MEM) load_pump<L>(h, row, t);
+  }
+  // v = row * FFT(v)
+  template <class TW>
+  __device__ __forceinline__ void after_fft(cplx (&v)[8], cplx* buf, int t, const TW& tw) const {
+    if constexpr (MEM) {
+      cplx g[8];
+      fft_field1<L, false, kWaveFft<L>>(v, buf, t, tw,
+                                        [&]() __attribute__((always_inline)) { load_pump<L>(g, src, t); });
+#pragma unroll
+      for (int m = 0; m < 8; m++) v[m] = v[m] * g[m];
+    } else {
+      fft_field1<L, false, kWaveFft<L>>(v, buf, t, tw);
+#pragma unroll
+      for (int m = 0; m < 8; m++) v[m] = v[m] * h[m];
+    }
+  }
+  __device__ __forceinline__ cplx at(int m, int t) const { return MEM ? src[t + FftShape<L>::T * m] : h[MEM ? 0 : m]; }
+};
+
+// FFT(k) of a stage, k = IFFT( FFT( IFFT(FFT(r |y|^2) * R) * y ) * (nl0 + nl1*omega) ), from
+// y N (an inverse transform left unscaled) and r / N^4: k is cubic in y and passes one more
+// inverse transform.
+template <int L, class ROW, class TW>
+__device__ __forceinline__ void gnlse_stage(const cplx (&y)[8], double r, cplx (&k)[8], const ROW& ram, const ROW& flt,
+                                            cplx* buf, int t, const TW& tw) {
 #pragma unroll
   for (int m = 0; m < 8; m++) k[m] = mk(r * abs2(y[m]), 0.0);
-  fft_field1<L, false, kWaveFft<L>>(k, buf, t, tw);
-#pragma unroll
-  for (int m = 0; m < 8; m++) k[m] = k[m] * ram[m];
+  ram.after_fft(k, buf, t, tw);
   fft_field1<L, true, kWaveFft<L>>(k, buf, t, tw);
-  scale_inv<L>(k);
 #pragma unroll
   for (int m = 0; m < 8; m++) k[m] = k[m] * y[m];
-  fft_field1<L, false, kWaveFft<L>>(k, buf, t, tw);
-#pragma unroll
-  for (int m = 0; m < 8; m++) k[m] = k[m] * flt[m];
-  fft_field1<L, true, kWaveFft<L>>(k, buf, t, tw);
-  scale_inv<L>(k);
+  flt.after_fft(k, buf, t, tw);
 }
 
-// One Chi3GNLSE propagation of field `field` on the T lanes that hold it.
+// One Chi3GNLSE propagation of field `field` on the T lanes that hold it.  The state and
+// the RK4 sum are kept as spectra: a stage ends in the spectrum of k, the next input is one
+// inverse transform of a + h k, and the last stage goes straight on to the dispersion
+// phase, 16 transforms per step where the time-domain state takes 18.  The transforms bound
+// the step (one wave per SIMD, their exchanges and arithmetic in turn); the factors 1/N, powers
+// of two, are all in r.  64 rows, N = 2048, 199 steps: 5.73 -> 5.30 ms; N = 4096, 49
+// steps: 5.70 -> 4.50, there also as the rows no longer sit in registers across transforms.
 template <int L>
 __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool active, int t, cplx* buf,
                                             const cplx* twl) {
   using F = FftShape<L>;
-  constexpr int N = F::N, T = F::T;
+  constexpr int N = F::N;
+  constexpr double inv4 = 1.0 / ((double)N * N * N * N);
   typename PropTw<L>::type tw;
   init_twiddles<L>(tw, kp.tw, twl, t);
-  cplx ds[8], ram[8], flt[8];
-#pragma unroll
-  for (int m = 0; m < 8; m++) {
-    ds[m] = kp.dstep[t + T * m];
-    ram[m] = kp.raman[t + T * m];
-    flt[m] = kp.filt[t + T * m];
-  }
+  SpectralRow<L, PropTw<L>::LEAN> ds, ram, flt;
+  ds.init(kp.dstep, t);
+  ram.init(kp.raman, t);
+  flt.init(kp.filt, t);
 
-  cplx a[1][8];
+  cplx a[1][8], y[8];  // a: spectrum; y: N times the time-domain stage input
   load_inputs<L, 1>(a, kp, field, t, active);
   prologue<L, 1>(a, kp, buf, t, tw, field, active);
   if (kp.nZ > 1) {
-    fft_field1<L, true, kWaveFft<L>>(a[0], buf, t, tw);
-    scale_inv<L>(a[0]);
-    if (kp.kind == KIND_GRID) store_row<L>(grid_row(kp, kp.gridT, field, 1, 0, 0, N), a[0], t, active);
+#pragma unroll
+    for (int m = 0; m < 8; m++) y[m] = a[0][m];
+    fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
+    if (kp.kind == KIND_GRID) store_scaled<L>(grid_row(kp, kp.gridT, field, 1, 0, 0, N), y, t, active);
   }
 
   for (int i = 1; i < kp.nZ; i++) {
     const cplx* c = kp.coef + (size_t)i * 3;
-    const double r0 = c[0].re, r1 = c[1].re, r2 = c[2].re;
-    // acc accumulates ((k1 + 2 k2) + 2 k3) + k4 in the reference's order
-    cplx y[8], k[8], acc[8];
-    gnlse_stage<L>(a[0], r0, k, ram, flt, buf, t, tw);
+    const double r0 = c[0].re * inv4, r1 = c[1].re * inv4, r2 = c[2].re * inv4;
+    cplx k[8], acc[8];
+    gnlse_stage<L>(y, r0, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
       acc[m] = k[m];
       y[m] = a[0][m] + 0.5 * k[m];
     }
+    fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
     gnlse_stage<L>(y, r1, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
       acc[m] = acc[m] + 2.0 * k[m];
       y[m] = a[0][m] + 0.5 * k[m];
     }
+    fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
     gnlse_stage<L>(y, r1, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
       acc[m] = acc[m] + 2.0 * k[m];
       y[m] = a[0][m] + k[m];
     }
+    fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
     gnlse_stage<L>(y, r2, k, ram, flt, buf, t, tw);
 #pragma unroll
-    for (int m = 0; m < 8; m++) a[0][m] = a[0][m] + (acc[m] + k[m]) * (1. / 6.);
-
-    fft_field1<L, false, kWaveFft<L>>(a[0], buf, t, tw);
-#pragma unroll
-    for (int m = 0; m < 8; m++) a[0][m] = a[0][m] * ds[m];
+    for (int m = 0; m < 8; m++) {
+      a[0][m] = (a[0][m] + (acc[m] + k[m]) * (1. / 6.)) * ds.at(m, t);
+      y[m] = a[0][m];
+    }
     if (i < kp.nZ - 1) {
       if (kp.kind == KIND_GRID) store_row<L>(grid_row(kp, kp.gridF, field, 1, 0, i, N), a[0], t, active);
-      fft_field1<L, true, kWaveFft<L>>(a[0], buf, t, tw);
-      scale_inv<L>(a[0]);
-      if (kp.kind == KIND_GRID) store_row<L>(grid_row(kp, kp.gridT, field, 1, 0, i, N), a[0], t, active);
+      fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
+      if (kp.kind == KIND_GRID) store_scaled<L>(grid_row(kp, kp.gridT, field, 1, 0, i, N), y, t, active);
     }
   }
   epilogue<L, 1>(a, kp, buf, t, tw, field, active);

@@ -61,16 +61,6 @@ __device__ __forceinline__ void load_prop_row(cplx (&al)[8], cplx (&be)[8], cons
   }
 }
 
-template <int L>
-__device__ __forceinline__ void store_scaled(cplx* __restrict__ dst, const cplx (&v)[8], int t, bool active) {
-  constexpr int T = FftShape<L>::T;
-  constexpr double s = 1.0 / FftShape<L>::N;
-  if (active) {
-#pragma unroll
-    for (int m = 0; m < 8; m++) dst[t + T * m] = v[m] * s;
-  }
-}
-
 // Where the step's rows live, per size and launch.  MANY: more fields than one wave
 // per SIMD.
 //  Up to N = 512 (one wave per field): the propagator rows are fetched after the
