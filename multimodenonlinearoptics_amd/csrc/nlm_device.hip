@@ -425,6 +425,19 @@ void tic(nlm_plan* p, int slot) {
   if (p->timing) (void)hipEventRecord(p->ev[slot], p->stream);
 }
 
+// R[k] = conj(R[N-k]) to the rounding of the transform that made R
+static bool hermitian(const cplx* R, int N) {
+  double top = 0, off = 0;
+  for (int k = 0; k < N; k++) {
+    const cplx a = R[k], b = R[k ? N - k : 0];
+    top = std::max(top, std::max(std::fabs(a.re), std::fabs(a.im)));
+    const double d = std::max(std::fabs(a.re - b.re), std::fabs(a.im + b.im));
+    if (d != d) return false;
+    off = std::max(off, d);
+  }
+  return off <= 64 * 2.220446049250313e-16 * top;
+}
+
 extern "C" int nlm_plan_create(const nlm_plan_desc* d, nlm_plan** out) {
   *out = nullptr;
   if (!d) return set_err(NLM_INVALID_ARGUMENT, "null plan descriptor");
@@ -473,6 +486,7 @@ extern "C" int nlm_plan_create(const nlm_plan_desc* d, nlm_plan** out) {
   if (p->model == NLM_CHI3GNLSE) {
     if ((e = upload(p->raman, d->raman, p->N, p->stream))) return fail(e);
     if ((e = upload(p->filt, d->gnlse_filter, p->N, p->stream))) return fail(e);
+    p->ramanReal = hermitian((const cplx*)d->raman, p->N) ? 1 : 0;
   }
   if (hipStreamSynchronize(p->stream) != hipSuccess) return fail(set_err(NLM_DEVICE_ERROR, "upload failed"));
   *out = p;
@@ -956,7 +970,7 @@ static int batch_common(nlm_plan* p, const cplx* in_dev, int rows, int cols, int
   }
   input_channels(p->nS, cols / N, input_mode, kp.inPos);
   if (rows == 0) return NLM_OK;
-  if (nlm_big_supported(p->model, p->L)) {
+  if (nlm_big_supported(p->model, p->L) || nlm_big_better(p)) {
     tic(p, 2);
     if (int e = nlm_big_batch(p, in_dev, rows, cols, in_time, kp.inPos[0] < 0 ? 0 : kp.inPos[0], n_out,
                               kp.outPos[0] < 0 ? 0 : kp.outPos[0], out_dev))

@@ -81,6 +81,7 @@ struct nlm_plan_s {
   DevBuf<cplx> cascade[2][2];  // products of nlm_greens_cascade whose last plan this is
   // staged transform for Chi3GNLSE with nFreqs > 8192 (nlm_big.hip)
   DevBuf<cplx> bigState, bigH;
+  int ramanReal = 0;  // the Raman response is the spectrum of a real one
   DevBuf<int> bigBase;
   hipGraphExec_t bigExec = nullptr;
   int bigKey[6] = {0, 0, 0, 0, 0, 0};
@@ -114,6 +115,8 @@ int get_twiddles(int n, const cplx** out);
 void input_channels(int nS, int nCh, int inputMode, int* inPos);
 // Chi3GNLSE batches with nFreqs 16384 / 32768 (nlm_big.hip)
 bool nlm_big_supported(int model, int L);
+// 8192, whose batches run staged too although one workgroup could hold a field
+bool nlm_big_better(const nlm_plan_s* p);
 int nlm_big_batch(nlm_plan_s* p, const cplx* in, int rows, int cols, int inTime, int inPos, int nOut, int outPos,
                   cplx* out);
 // Any even nFreqs outside the power-of-two kernels (nlm_any.hip): not a power of

@@ -450,7 +450,7 @@ struct SpectralRow {
     if constexpr (MEM) {
       cplx g[8];
       fft_field1<L, false, kWaveFft<L>>(v, buf, t, tw,
-                                        [&]() __attribute__((always_inline)) { load_pump<L>(g, src, t); });
+                                        [&]() __attribute__((always_inline)) { load_pump<L>(g, src, opaque_lane(t)); });
 #pragma unroll
       for (int m = 0; m < 8; m++) v[m] = v[m] * g[m];
     } else {
@@ -483,14 +483,18 @@ __device__ __forceinline__ void gnlse_stage(const cplx (&y)[8], double r, cplx (
 // phase, 16 transforms per step where the time-domain state takes 18.  The transforms bound
 // the step (one wave per SIMD, their exchanges and arithmetic in turn); the factors 1/N, powers
 // of two, are all in r.  64 rows, N = 2048, 199 steps: 5.73 -> 5.30 ms; N = 4096, 49
-// steps: 5.70 -> 4.50, there also as the rows no longer sit in registers across transforms.
+// steps: 5.70 -> 3.43.  Up to N = 2048 rows and addresses stay in registers, AGPRs included
+// (fetched and formed per stage: 5.66 ms).
 template <int L>
-__device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool active, int t, cplx* buf,
+__device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool active, int t0, cplx* buf,
                                             const cplx* twl) {
   using F = FftShape<L>;
   constexpr int N = F::N;
+  int t = t0;
   constexpr double inv4 = 1.0 / ((double)N * N * N * N);
-  typename PropTw<L>::type tw;
+  // N = 4096: with the rows fetched and addresses formed per stage the twiddles fit registers
+  // (with rows and addresses held and twiddles in LDS 92 us per step of 64 rows, so 70)
+  typename std::conditional<FftShape<L>::LOG == 12, RegTwiddles<L>, typename PropTw<L>::type>::type tw;
   init_twiddles<L>(tw, kp.tw, twl, t);
   SpectralRow<L, PropTw<L>::LEAN> ds, ram, flt;
   ds.init(kp.dstep, t);
@@ -508,6 +512,7 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool a
   }
 
   for (int i = 1; i < kp.nZ; i++) {
+    if (PropTw<L>::LEAN) t = opaque_lane(t0);
     const cplx* c = kp.coef + (size_t)i * 3;
     const double r0 = c[0].re * inv4, r1 = c[1].re * inv4, r2 = c[2].re * inv4;
     cplx k[8], acc[8];
@@ -518,6 +523,7 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool a
       y[m] = a[0][m] + 0.5 * k[m];
     }
     fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
+    if (PropTw<L>::LEAN) t = opaque_lane(t0);
     gnlse_stage<L>(y, r1, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
@@ -525,6 +531,7 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool a
       y[m] = a[0][m] + 0.5 * k[m];
     }
     fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
+    if (PropTw<L>::LEAN) t = opaque_lane(t0);
     gnlse_stage<L>(y, r1, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
@@ -532,6 +539,7 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool a
       y[m] = a[0][m] + k[m];
     }
     fft_field1<L, true, kWaveFft<L>>(y, buf, t, tw);
+    if (PropTw<L>::LEAN) t = opaque_lane(t0);
     gnlse_stage<L>(y, r2, k, ram, flt, buf, t, tw);
 #pragma unroll
     for (int m = 0; m < 8; m++) {
