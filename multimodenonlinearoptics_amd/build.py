@@ -72,12 +72,12 @@ def build(force=False, jobs=None, verbose=False):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_big.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_multi.o")
     objs.append(o)
-    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_quad.hpp", "nlm_internal.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_multi_stage.o")
     objs.append(o)
-    deps = _deps("nlm_multi_stage.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", *dev_hdrs)
+    deps = _deps("nlm_multi_stage.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi_stage.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_compose.o")
@@ -103,14 +103,14 @@ def build(force=False, jobs=None, verbose=False):
     for v in range(4):  # FFT schedule variants of the step-table kernel (chosen by the autotuner)
         o = os.path.join(OBJ, "nlm_prop_tab_v%d.o" % v)
         objs.append(o)
-        deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", *dev_hdrs)
+        deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_TAB_VARIANT=%d" % v, "-c",
                                                 os.path.join(CSRC, "nlm_prop_tab.hip"), "-o", o])
     # the single-wave sizes of the step-table kernel, with the memory-clause scheduler
     o = os.path.join(OBJ, "nlm_prop_tab_small.o")
     objs.append(o)
-    deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", *dev_hdrs)
+    deps = _deps("nlm_prop_tab.hip", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause", "-DNLM_TAB_SMALL",
                                             "-c", os.path.join(CSRC, "nlm_prop_tab.hip"), "-o", o])
@@ -124,7 +124,7 @@ def build(force=False, jobs=None, verbose=False):
     for m in PROP_MODELS:  # heterogeneous-batch kernels of each model
         o = os.path.join(OBJ, "nlm_multi_%d.o" % m)
         objs.append(o)
-        deps = _deps("nlm_multi_inst.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", *dev_hdrs)
+        deps = _deps("nlm_multi_inst.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
         if force or _stale(o, deps):
             steps.append([HIPCC] + HIP_FLAGS + ["-DNLM_INST_MODEL=%d" % m, "-c",
                                                 os.path.join(CSRC, "nlm_multi_inst.hip"), "-o", o])

@@ -16,7 +16,7 @@
 // Green's impulses or batch rows.  The propagator also absorbs the inverse
 // transform's 1/N (an exact power of two), so the field between steps is kept
 // unscaled.
-#include "nlm_tab.hpp"
+#include "nlm_quad.hpp"
 
 // tab[(i*N + k)*2 + {0,1}] = {(Re R(1), Re R(i)), (Im R(1), Im R(i))} * scale for
 // steps i = 1..nZ-1: Re x' = p.re Re x + p.im Im x, Im x' = q.re Re x + q.im Im x.
@@ -97,6 +97,19 @@ prop_fn nlm_pick_prop_tab_small(int L) {
     case 7: return &launch_prop_tab<7>;
     case 8: return &launch_prop_tab<8>;
     case 9: return &launch_prop_tab<9>;
+  }
+  return nullptr;
+}
+
+// Four points per lane, nFreqs 8..256.
+prop_fn nlm_pick_prop_quad(int L) {
+  switch (L) {
+    case 3: return &quad::launch<3>;
+    case 4: return &quad::launch<4>;
+    case 5: return &quad::launch<5>;
+    case 6: return &quad::launch<6>;
+    case 7: return &quad::launch<7>;
+    case 8: return &quad::launch<8>;
   }
   return nullptr;
 }
