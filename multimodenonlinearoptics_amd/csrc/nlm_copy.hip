@@ -2,12 +2,13 @@
 //
 // hipMemcpy to pageable memory goes through the runtime's own staging, one thread
 // filling the destination: 17.8 GB/s measured for 128 MB, and less into freshly
-// allocated pages, against 56.8 GB/s into pinned memory.  Here large copies run
-// through a pinned staging area in 1 MB pieces, two per participant in flight, and the
-// caller and up to three helper threads move the pieces between the staging area and
-// the destination.  That pays from a few megabytes (below, waking the helpers costs more
-// than they save: 2 MB each way 50 us slower).  Small results are gathered in the
-// area and share one wait; between the two the runtime's own copy is used.
+// allocated pages, against 56.8 GB/s into pinned memory.  Here large results run through a
+// pinned staging area in 1 MB pieces, two per participant in flight, and the caller and up to
+// three helper threads move the pieces to the destination.  That pays from about 3 MB (a
+// batch's result of 6.2 MB 816 -> 766 us for the call, 12.5 MB 2.24 -> 1.35 ms, two of 16 MB 2.02 ->
+// 1.28; at 2 MB 50 us slower).  Small results are gathered in the area and share one wait;
+// between the two the runtime's own copy is used, as for every upload, whose source pages are
+// there already (in pieces by the helpers a 6.2 MB input made the call 766 -> 1395 us).
 // Calls, ms before -> now: Chi2PDC Green's N = 512 (C, S of 4 MB each) 2.63 -> 2.37, N =
 // 32 0.116 -> 0.080; Chi3 z-grids N = 512, nZ = 1000 (48 MB) 11.4 -> 10.6.
 #include <sys/types.h>
@@ -149,7 +150,7 @@ Helpers& helpers() {
 
 // One participant's share of a large copy: pieces part, part + parts, ..., alternating
 // between its two slots.
-hipError_t share(Staging* st, char* host, char* dev, size_t bytes, bool toHost, int part, int parts, hipStream_t s) {
+hipError_t share(Staging* st, char* host, const char* dev, size_t bytes, int part, int parts, hipStream_t s) {
   const size_t n = (bytes + PIECE - 1) / PIECE;
   const auto len = [&](size_t c) { return std::min(PIECE, bytes - c * PIECE); };
   hipError_t e = hipSuccess;
@@ -161,23 +162,18 @@ hipError_t share(Staging* st, char* host, char* dev, size_t bytes, bool toHost, 
     if (pending[k] < n) {  // the piece this slot still holds
       e = hipEventSynchronize(st->ev[q]);
       if (e != hipSuccess) break;
-      if (toHost) memcpy(host + pending[k] * PIECE, st->slot(q), len(pending[k]));
+      memcpy(host + pending[k] * PIECE, st->slot(q), len(pending[k]));
       pending[k] = n;
     }
     if (c >= n) continue;
-    if (toHost) {
-      e = hipMemcpyAsync(st->slot(q), dev + c * PIECE, len(c), hipMemcpyDeviceToHost, s);
-    } else {
-      memcpy(st->slot(q), host + c * PIECE, len(c));
-      e = hipMemcpyAsync(dev + c * PIECE, st->slot(q), len(c), hipMemcpyHostToDevice, s);
-    }
+    e = hipMemcpyAsync(st->slot(q), dev + c * PIECE, len(c), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipEventRecord(st->ev[q], s);
     pending[k] = c;
   }
   return e;
 }
 
-hipError_t large(Staging* st, char* host, char* dev, size_t bytes, bool toHost, hipStream_t s) {
+hipError_t large(Staging* st, char* host, const char* dev, size_t bytes, hipStream_t s) {
   hipError_t errs[PARTS] = {};
   const int device = st->device;
   const std::function<void(int)> body = [&](int part) {
@@ -185,9 +181,9 @@ hipError_t large(Staging* st, char* host, char* dev, size_t bytes, bool toHost, 
       errs[part] = hipSetDevice(device);
       if (errs[part] != hipSuccess) return;
     }
-    errs[part] = share(st, host, dev, bytes, toHost, part, PARTS, s);
+    errs[part] = share(st, host, dev, bytes, part, PARTS, s);
   };
-  if (!helpers().run(body)) return share(st, host, dev, bytes, toHost, 0, 1, s);
+  if (!helpers().run(body)) return share(st, host, dev, bytes, 0, 1, s);
   for (hipError_t e : errs)
     if (e != hipSuccess) return e;
   return hipSuccess;
@@ -223,7 +219,7 @@ int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
     if (c.bytes >= LARGE) {
       flush(i);
       first = i + 1;
-      if (e == hipSuccess) e = large(st, (char*)c.host, (char*)const_cast<void*>(c.dev), c.bytes, true, s);
+      if (e == hipSuccess) e = large(st, (char*)c.host, (const char*)c.dev, c.bytes, s);
     } else if (c.bytes > SMALL) {
       e = hipMemcpyAsync(c.host, c.dev, c.bytes, hipMemcpyDeviceToHost, s);
     } else {
@@ -244,21 +240,8 @@ int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
 
 int nlm_to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
   if (bytes == 0) return NLM_OK;
-  if (bytes < LARGE) {  // the runtime has taken its copy when the call returns
-    const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
-    return e == hipSuccess ? NLM_OK : failed(e);
-  }
-  Staging* st = nullptr;
-  hipError_t e = take(&st);
-  if (e != hipSuccess) return failed(e);
-  e = large(st, (char*)const_cast<void*>(host), (char*)dev, bytes, false, s);
-  if (e != hipSuccess) {
-    (void)hipStreamSynchronize(s);
-    st->destroy();
-    return failed(e);
-  }
-  give(st);
-  return NLM_OK;
+  const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
+  return e == hipSuccess ? NLM_OK : failed(e);
 }
 
 bool nlm_on_device(const void* ptr, int device) {
