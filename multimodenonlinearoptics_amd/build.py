@@ -57,7 +57,7 @@ def build(force=False, jobs=None, verbose=False):
     objs = []
     o = os.path.join(OBJ, "nlm_device.o")
     objs.append(o)
-    deps = _deps("nlm_device.hip", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_device.hip", "nlm_internal.hpp", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_device.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_adjoint.o")

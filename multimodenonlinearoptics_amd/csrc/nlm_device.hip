@@ -27,6 +27,7 @@
 
 #include "../../include/nlm.h"
 #include "nlm_internal.hpp"
+#include "nlm_quad.hpp"
 
 // ---------------------------------------------------------------------------
 // errors
@@ -317,7 +318,10 @@ static void launch_pump_linear(const cplx* F0, const cplx* env, const double* Dp
 template <int L>
 static void launch_pump_chi3(const cplx* env, const double* Dp, double dzp, const cplx* dsp, const cplx* relI,
                              int nZP, cplx* pF, cplx* pT, const cplx* tw, hipStream_t s) {
-  hipLaunchKernelGGL((k_pump_chi3<L>), dim3(1), dim3(FftShape<L>::T), 0, s, env, Dp, dzp, dsp, relI, nZP, pF, pT, tw);
+  if constexpr (L <= 8)
+    hipLaunchKernelGGL((quad::k_pump_chi3<L>), dim3(1), dim3(quad::Shape<L>::T), 0, s, env, Dp, dzp, dsp, relI, nZP, pF, pT, tw);
+  else
+    hipLaunchKernelGGL((k_pump_chi3<L>), dim3(1), dim3(FftShape<L>::T), 0, s, env, Dp, dzp, dsp, relI, nZP, pF, pT, tw);
 }
 template <int L>
 static void launch_fft(const cplx* in, cplx* out, int count, const cplx* tw, bool inv, hipStream_t s) {

@@ -11,11 +11,12 @@ static prop_fn pick_L() {
   if constexpr (MODEL == NLM_CHI3GNLSE) return &launch_gnlse<L>;
   else {
     using M = typename ModelOf<MODEL>::type;
-    if constexpr (M::NS > 1)
-      if constexpr (modes::Pow2<L, M::NS>::OK) {
-        return &modes::launch_prop_modes<M, L>;
-      }
-    return &launch_prop<M, L>;
+    constexpr bool groups = [] {
+      if constexpr (M::NS > 1) return modes::Pow2<L, M::NS>::OK;
+      else return false;
+    }();
+    if constexpr (groups) return &modes::launch_prop_modes<M, L>;
+    else return &launch_prop<M, L>;
   }
 }
 

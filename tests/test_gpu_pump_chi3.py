@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 TOL = 1e-10
 
 
-@pytest.mark.parametrize("N", [8, 64, 512, 1024, 4096, 90, 600])
+@pytest.mark.parametrize("N", [8, 16, 32, 64, 128, 256, 512, 1024, 4096, 90, 600])
 @pytest.mark.parametrize("phase", [0.05, 0.785, 2.0])
 def test_pump_rows(nlm, oracle, N, phase):
     print("pump N=%d phase=%g" % (N, phase), flush=True)
