@@ -6,7 +6,8 @@
 // Four points per lane instead of eight halve the arithmetic of that chain and use twice the
 // waves; a transform of N = 2^L takes radix 4 stages and one of radix 2 if L is odd, at most
 // one exchange more.  A field is at most one wave (N <= 256), so the exchanges are ordered
-// within the wave.  Calls of 200 steps, us (eight points -> four): signal N = 32
+// within the wave; with barriers between several waves the form loses (one field, 199 steps: N = 512
+// 415 -> 450 us, 1024 531 -> 594; Chi3 pump N = 512 2.25 -> 2.32 us per row).  Calls of 200 steps, us (eight points -> four): signal N = 32
 // 256 -> 194, 64 275 -> 203, 256 370 -> 262; Green's N = 16 261 -> 151, 32 238 -> 193, 64 283 ->
 // 226, 256 504 -> 470 (of which the rows fetched two steps ahead instead of one: 5 %, 20 % at 256).
 #pragma once
