@@ -651,11 +651,17 @@ void launch_adjoint_segment(const Stager& sg, const BigParams& bp, int i0, int i
     }
 }
 
+int ensure_state(nlm_plan* p, int rows) {
+  int e;
+  if ((e = p->bigState.ensure(5 * (size_t)rows * p->N)) || (e = p->bigH.ensure(5 * (size_t)p->N))) return e;
+  return p->bigBase.ensure(1);
+}
+
 int setup_params(nlm_plan* p, const Stager& sg, int rows, BigParams& bp) {
   const int N = p->N;
   const size_t BN = (size_t)rows * N;
   int e;
-  if ((e = p->bigState.ensure(5 * BN)) || (e = p->bigH.ensure(5 * (size_t)N)) || (e = p->bigBase.ensure(1))) return e;
+  if ((e = ensure_state(p, rows))) return e;
   const cplx* twM = nullptr;
   if ((e = get_twiddles(1 << sg.LM, &twM))) return e;
   hipLaunchKernelGGL(k_big_perm, dim3((N + 255) / 256), dim3(256), 0, p->stream, p->raman.p, p->filt.p, p->dstep.p,
@@ -692,12 +698,18 @@ bool nlm_big_supported(int model, int L) { return model == NLM_CHI3GNLSE && (L =
 
 // N = 8192 also fits one workgroup's LDS, with 1024 lanes of 128 registers that spill and one
 // CU per row: 4 rows 307 us per step against 72 staged, 64 rows 385 against 148, 128 rows 424
-// against 246.  At N = 4096 the in-LDS kernel is the faster one (4 rows 55 against 61, 64 rows
-// 70 against 95).  Under a caller's stream capture the in-LDS kernel, one plain launch, stays.
-bool nlm_big_better(const nlm_plan* p) {
-  if (p->model != NLM_CHI3GNLSE || p->L != 13 || p->nZ < 2) return false;
+// against 246, 256 rows about 430 against 391.  With more rows than CUs the two are close, and
+// the in-LDS kernel needs no state arrays in memory; it also runs when these do not fit, and
+// under a caller's stream capture, where it is one plain launch.  At N = 4096 it is the faster
+// one (4 rows 55 against 61, 64 rows 70 against 95).
+bool nlm_big_better(nlm_plan* p, int rows) {
+  constexpr int CUS = 256;
+  if (p->model != NLM_CHI3GNLSE || p->L != 13 || p->nZ < 2 || rows > CUS) return false;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(p->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(p->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+  if (ensure_state(p, rows) == NLM_OK) return true;
+  (void)hipGetLastError();
+  return false;
 }
 
 // Batch propagation of a Chi3GNLSE plan with nFreqs 16384 or 32768 (see above).

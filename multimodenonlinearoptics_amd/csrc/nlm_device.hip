@@ -977,7 +977,7 @@ static int batch_common(nlm_plan* p, const cplx* in_dev, int rows, int cols, int
   }
   input_channels(p->nS, cols / N, input_mode, kp.inPos);
   if (rows == 0) return NLM_OK;
-  if (nlm_big_supported(p->model, p->L) || nlm_big_better(p)) {
+  if (nlm_big_supported(p->model, p->L) || nlm_big_better(p, rows)) {
     tic(p, 2);
     if (int e = nlm_big_batch(p, in_dev, rows, cols, in_time, kp.inPos[0] < 0 ? 0 : kp.inPos[0], n_out,
                               kp.outPos[0] < 0 ? 0 : kp.outPos[0], out_dev))

@@ -116,7 +116,7 @@ void input_channels(int nS, int nCh, int inputMode, int* inPos);
 // Chi3GNLSE batches with nFreqs 16384 / 32768 (nlm_big.hip)
 bool nlm_big_supported(int model, int L);
 // 8192, whose batches run staged too although one workgroup could hold a field
-bool nlm_big_better(const nlm_plan_s* p);
+bool nlm_big_better(nlm_plan_s* p, int rows);
 int nlm_big_batch(nlm_plan_s* p, const cplx* in, int rows, int cols, int inTime, int inPos, int nOut, int outPos,
                   cplx* out);
 // Any even nFreqs outside the power-of-two kernels (nlm_any.hip): not a power of
