@@ -82,7 +82,7 @@ enum Table { TAB_RAMAN = 0, TAB_FILTER, TAB_DISP, TAB_IN, TAB_DISP_OUT };
 struct BigParams {
   int B, nSteps, N, P, LM;  // N = P 2^LM
   int real;                 // real Raman convolution
-  const int* base;          // current first step of the replayed graph
+  const BigArgs* args;      // of the replayed graph
   cplx* A;                  // [B][P][M] spectrum of the state
   cplx* ACC;                // [B][P][M] spectrum of a + (k1 + 2 k2 + 2 k3) / 6
   cplx* Y;                  // [B][N] stage input y (time, natural order)
@@ -94,7 +94,7 @@ struct BigParams {
   const cplx* coef;         // [nZ][3], .re = relative intensity of the stage
   const cplx* in;           // [B][inCols]
   int inCols, inPos;
-  cplx* out;                // [B][nOut*N] or nullptr (recomputation)
+  cplx* out;                // [B][nOut*N] or nullptr (recomputation); a replay's is in args
   int nOut, outPos, outTime;
   // checkpoints [B][nSeg][P][M] of the spectra of the states a_{sK}
   cplx* ckpt;
@@ -112,7 +112,10 @@ struct BigParams {
 };
 
 __device__ __forceinline__ int step_of(const BigParams& bp, int di, int fixedStep) {
-  return fixedStep >= 0 ? fixedStep : *bp.base + di;
+  return fixedStep >= 0 ? fixedStep : bp.args->step + di;
+}
+__device__ __forceinline__ cplx* out_of(const BigParams& bp, int fixedStep) {
+  return fixedStep >= 0 ? bp.out : bp.args->out;
 }
 
 __device__ __forceinline__ bool seg_has(const BigParams& bp, int i) {
@@ -285,10 +288,11 @@ __global__ void __launch_bounds__(MIX_THREADS) k_big_mix(BigParams bp, int mode,
     case MIX_STATE: {
       const bool state = kind == MIX_STATE;
       if (state && i == bp.nSteps) {
-        if (bp.out && bp.outTime) {
+        cplx* out = out_of(bp, fixedStep);
+        if (out && bp.outTime) {
 #pragma unroll
           for (int n1 = 0; n1 < P; n1++)
-            bp.out[(size_t)f * bp.nOut * N + (size_t)bp.outPos * N + n1 * M + n2] = v[n1];
+            out[(size_t)f * bp.nOut * N + (size_t)bp.outPos * N + n1 * M + n2] = v[n1];
         }
         return;
       }
@@ -424,9 +428,9 @@ __global__ void __launch_bounds__((FftShape<LM>::T), (2)) k_big_conv(BigParams b
 #pragma unroll
       for (int m = 0; m < 8; m++) v[m] = (c[m] + (v[m] * h[m]) * (1. / 6.)) * D[t + T * m];
       if (last && !bp.outTime) {
-        if (bp.out) {
+        if (cplx* out = out_of(bp, fixedStep)) {
 #pragma unroll
-          for (int m = 0; m < 8; m++) bp.out[(size_t)f * bp.nOut * N + (size_t)bp.outPos * N + at(m)] = v[m];
+          for (int m = 0; m < 8; m++) out[(size_t)f * bp.nOut * N + (size_t)bp.outPos * N + at(m)] = v[m];
         }
         return;
       }
@@ -534,8 +538,11 @@ __global__ void __launch_bounds__((FftShape<LM>::T), (2)) k_big_conv(BigParams b
   }
 }
 
-__global__ void k_big_set_base(int* base, int value, int add) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) base[0] = add ? base[0] + value : value;
+__global__ void k_big_set_args(BigArgs* a, BigArgs value) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *a = value;
+}
+__global__ void k_big_advance(BigArgs* a, int steps) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) a->step += steps;
 }
 
 // Hp[tab][k1 M + k2] = H[k1 + P k2]  (tab 4: disp * halfOut)
@@ -654,7 +661,7 @@ void launch_adjoint_segment(const Stager& sg, const BigParams& bp, int i0, int i
 int ensure_state(nlm_plan* p, int rows) {
   int e;
   if ((e = p->bigState.ensure(5 * (size_t)rows * p->N)) || (e = p->bigH.ensure(5 * (size_t)p->N))) return e;
-  return p->bigBase.ensure(1);
+  return p->bigArgs.ensure(1);
 }
 
 int setup_params(nlm_plan* p, const Stager& sg, int rows, BigParams& bp) {
@@ -674,7 +681,7 @@ int setup_params(nlm_plan* p, const Stager& sg, int rows, BigParams& bp) {
   bp.P = sg.P;
   bp.LM = sg.LM;
   bp.real = p->ramanReal;
-  bp.base = p->bigBase.p;
+  bp.args = p->bigArgs.p;
   bp.A = p->bigState.p;
   bp.Y = bp.A + BN;
   bp.ACC = bp.Y + BN;
@@ -732,11 +739,13 @@ int nlm_big_batch(nlm_plan* p, const cplx* in, int rows, int cols, int inTime, i
   bp.outTime = inTime;
   launch_prologue(sg, bp, inTime != 0, p->stream);
   HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_big_set_base, dim3(1), dim3(64), 0, p->stream, p->bigBase.p, 1, 0);
+  hipLaunchKernelGGL(k_big_set_args, dim3(1), dim3(64), 0, p->stream, p->bigArgs.p, BigArgs{1, out});
   HIP_TRY(hipGetLastError());
 
-  // the z loop: a graph of BIG_GRAPH_STEPS steps, rebuilt when its arguments
-  // change; NLM_NO_GRAPH=1 in the environment launches the same kernels
+  // the z loop: a graph of BIG_GRAPH_STEPS steps, rebuilt when the batch's shape or domain
+  // changes.  The caller's output buffer is an argument in device memory, not of the graph:
+  // 64 rows N = 8192, 32 steps into another buffer than the call before, 5.1 ms with the graph
+  // rebuilt (up to 8.4), 4.0 so.  NLM_NO_GRAPH=1 in the environment launches the same kernels
   // directly (for tools that do not follow graph launches)
   const int launches = (p->nZ - 1 + BIG_GRAPH_STEPS - 1) / BIG_GRAPH_STEPS;
   const int G = (p->nZ - 1 + launches - 1) / launches;  // fewest idle steps in the last replay
@@ -744,20 +753,25 @@ int nlm_big_batch(nlm_plan* p, const cplx* in, int rows, int cols, int inTime, i
   if (noGraph && noGraph[0] == '1') {
     for (int r = 0; r < launches; r++) {
       for (int di = 0; di < G; di++) launch_step(sg, bp, di, -1, p->stream);
-      hipLaunchKernelGGL(k_big_set_base, dim3(1), dim3(64), 0, p->stream, p->bigBase.p, G, 1);
+      hipLaunchKernelGGL(k_big_advance, dim3(1), dim3(64), 0, p->stream, p->bigArgs.p, G);
     }
     HIP_TRY(hipGetLastError());
     return NLM_OK;
   }
   if (!p->bigExec || p->bigKey[0] != rows || p->bigKey[1] != cols || p->bigKey[2] != inTime ||
-      p->bigKey[3] != inPos || p->bigKey[4] != nOut || p->bigKey[5] != outPos || p->bigIn != in ||
-      p->bigOut != out || p->bigStatePtr != p->bigState.p) {
-    if (p->bigExec) (void)hipGraphExecDestroy(p->bigExec);
+      p->bigKey[3] != inPos || p->bigKey[4] != nOut || p->bigKey[5] != outPos || p->bigStatePtr != p->bigState.p) {
+    if (p->bigExec) {
+      // an asynchronous call before this one may still be replaying it
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(p->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
+        HIP_TRY(hipStreamSynchronize(p->stream));
+      (void)hipGraphExecDestroy(p->bigExec);
+    }
     p->bigExec = nullptr;
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(p->stream, hipStreamCaptureModeThreadLocal));
     for (int di = 0; di < G; di++) launch_step(sg, bp, di, -1, p->stream);
-    hipLaunchKernelGGL(k_big_set_base, dim3(1), dim3(64), 0, p->stream, p->bigBase.p, G, 1);
+    hipLaunchKernelGGL(k_big_advance, dim3(1), dim3(64), 0, p->stream, p->bigArgs.p, G);
     const hipError_t ce = hipGetLastError();
     const hipError_t ee = hipStreamEndCapture(p->stream, &g);
     if (ce != hipSuccess || ee != hipSuccess) {
@@ -773,8 +787,6 @@ int nlm_big_batch(nlm_plan* p, const cplx* in, int rows, int cols, int inTime, i
     }
     const int key[6] = {rows, cols, inTime, inPos, nOut, outPos};
     std::memcpy(p->bigKey, key, sizeof key);
-    p->bigIn = in;
-    p->bigOut = out;
     p->bigStatePtr = p->bigState.p;
   }
   for (int r = 0; r < launches; r++) HIP_TRY(hipGraphLaunch(p->bigExec, p->stream));

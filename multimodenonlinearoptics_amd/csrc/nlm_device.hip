@@ -510,7 +510,7 @@ extern "C" int nlm_plan_destroy(nlm_plan* p) {
   if (p->bigExec) (void)hipGraphExecDestroy(p->bigExec);
   p->bigState.release();
   p->bigH.release();
-  p->bigBase.release();
+  p->bigArgs.release();
   p->Dp.release();
   p->strength.release();
   for (auto& ev : p->ev)

@@ -59,6 +59,13 @@ int nlm_to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
 // whether ptr is memory of `device` that this process's HIP runtime knows
 bool nlm_on_device(const void* ptr, int device);
 
+// What a replay of the staged z loop reads from device memory (nlm_big.hip): its first step
+// and the caller's output.
+struct BigArgs {
+  int step;
+  cplx* out;
+};
+
 struct nlm_plan_s {
   int model = 0, N = 0, L = 0, nZ = 0, nS = 0, nP = 0, NC = 0, NCC = 0;
   int device = 0;
@@ -82,11 +89,9 @@ struct nlm_plan_s {
   // staged transform for Chi3GNLSE with nFreqs > 8192 (nlm_big.hip)
   DevBuf<cplx> bigState, bigH;
   int ramanReal = 0;  // the Raman response is the spectrum of a real one
-  DevBuf<int> bigBase;
+  DevBuf<BigArgs> bigArgs;
   hipGraphExec_t bigExec = nullptr;
   int bigKey[6] = {0, 0, 0, 0, 0, 0};
-  const void* bigIn = nullptr;
-  const void* bigOut = nullptr;
   const void* bigStatePtr = nullptr;
   DevBuf<cplx> anyScratch;  // workspaces of the any-length path (nlm_any.hip) when they exceed LDS
   DevBuf<cplx> stepTab;  // RK4 step propagators of one-mode undepleted media [nZ][N][2]
