@@ -89,7 +89,10 @@ int nlm_plan_create(const nlm_plan_desc* desc, nlm_plan** out);
 int nlm_plan_destroy(nlm_plan* plan);
 
 /* Run this plan's work on `hip_stream` (a hipStream_t); NULL restores the
- * plan's own stream.  Lets a caller order the engine against its own work. */
+ * plan's own stream.  Lets a caller order the engine against its own work.  A call
+ * that uses scratch of the plan waits on the device for the asynchronous one
+ * (nlm_batch_dev) that used it last, on whichever stream that was; everything else
+ * queued on the former stream is the caller's to order. */
 int nlm_plan_set_stream(nlm_plan* plan, void* hip_stream);
 void* nlm_plan_stream(nlm_plan* plan);
 

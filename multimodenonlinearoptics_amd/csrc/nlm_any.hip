@@ -481,6 +481,8 @@ int any_launch(nlm_plan_s* p, DevBuf<cplx>* own, int NS, int N, long items, AnyL
   if (!may_alloc && (!buf.p || buf.n < (size_t)out->grid * 2 * NS * N))
     return set_err(NLM_INVALID_ARGUMENT, "nFreqs " + std::to_string(N) +
                                              " needs a device workspace beyond LDS; use the allocating entry point");
+  if (p)
+    if (int e = scratch_wait(p)) return e;
   if (int e = buf.ensure((size_t)out->grid * 2 * NS * N)) return e;
   out->gws = buf.p;
   return NLM_OK;
@@ -543,6 +545,7 @@ int nlm_any_prop(nlm_plan_s* p, const KParams& kp, bool may_alloc) {
     if (int e = get_twiddles(p->N, &mp.tw)) return e;
     KParams kq = kp;
     if (oneMode) {
+      if (int e = scratch_wait(p)) return e;
       if (int e = p->stepTab.ensure((size_t)p->nZ * p->N * 2)) return e;
       nlm_launch_step_table(p->model, p->coef.p, p->cconst.p, p->pumpT[0].p, p->N, p->nZ, p->stepTab.p, p->stream);
       HIP_TRY(hipGetLastError());

@@ -668,7 +668,7 @@ int setup_params(nlm_plan* p, const Stager& sg, int rows, BigParams& bp) {
   const int N = p->N;
   const size_t BN = (size_t)rows * N;
   int e;
-  if ((e = ensure_state(p, rows))) return e;
+  if ((e = scratch_wait(p)) || (e = ensure_state(p, rows))) return e;
   const cplx* twM = nullptr;
   if ((e = get_twiddles(1 << sg.LM, &twM))) return e;
   hipLaunchKernelGGL(k_big_perm, dim3((N + 255) / 256), dim3(256), 0, p->stream, p->raman.p, p->filt.p, p->dstep.p,

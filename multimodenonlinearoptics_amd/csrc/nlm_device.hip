@@ -500,6 +500,10 @@ extern "C" int nlm_plan_create(const nlm_plan_desc* d, nlm_plan** out) {
 extern "C" int nlm_plan_destroy(nlm_plan* p) {
   if (!p) return NLM_OK;
   if (p->stream) (void)hipStreamSynchronize(p->stream);
+  if (p->scratchDone) {
+    if (p->scratchBusy) (void)hipEventSynchronize(p->scratchDone);
+    (void)hipEventDestroy(p->scratchDone);
+  }
   DevBuf<cplx>* bufs[] = {&p->dstep, &p->halfIn, &p->halfOut, &p->coef, &p->cconst, &p->raman, &p->filt,
                           &p->pumpT[0], &p->pumpT[1], &p->pumpF[0], &p->pumpF[1], &p->gridF, &p->gridT,
                           &p->G, &p->C, &p->S, &p->in, &p->out, &p->env, &p->F0, &p->dsp, &p->relI};
@@ -953,6 +957,27 @@ extern "C" int nlm_grid_download(nlm_plan* p, int mode, double* sf, double* st) 
   return nlm_to_host(out, 2, p->stream);
 }
 
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+int scratch_wait(nlm_plan* p) {
+  if (capturing(p->stream)) return NLM_OK;
+  p->scratchUsed = true;
+  if (p->scratchBusy) HIP_TRY(hipStreamWaitEvent(p->stream, p->scratchDone, 0));
+  return NLM_OK;
+}
+
+int scratch_mark(nlm_plan* p) {
+  if (!p->scratchUsed) return NLM_OK;
+  p->scratchUsed = false;
+  if (!p->scratchDone) HIP_TRY(hipEventCreateWithFlags(&p->scratchDone, hipEventDisableTiming));
+  HIP_TRY(hipEventRecord(p->scratchDone, p->stream));
+  p->scratchBusy = true;
+  return NLM_OK;
+}
+
 static int batch_common(nlm_plan* p, const cplx* in_dev, int rows, int cols, int in_time, int input_mode, int n_out,
                         const int32_t* outputs, cplx* out_dev) {
   const int N = p->N;
@@ -1007,7 +1032,10 @@ extern "C" int nlm_batch(nlm_plan* p, const double* inputs, int rows, int cols, 
 extern "C" int nlm_batch_dev(nlm_plan* p, const double* in_dev, int rows, int cols, int in_time, int input_mode,
                              int n_out, const int32_t* outputs, double* out_dev) {
   if (!p || !outputs || (rows > 0 && (!in_dev || !out_dev))) return set_err(NLM_INVALID_ARGUMENT, "null argument");
-  return batch_common(p, (const cplx*)in_dev, rows, cols, in_time, input_mode, n_out, outputs, (cplx*)out_dev);
+  p->scratchUsed = false;
+  const int e = batch_common(p, (const cplx*)in_dev, rows, cols, in_time, input_mode, n_out, outputs, (cplx*)out_dev);
+  const int m = scratch_mark(p);  // also after an error: part of the call may be queued
+  return e ? e : m;
 }
 
 extern "C" int nlm_greens(nlm_plan* p, int in_time, int n_in, const int32_t* inputs, int n_out, const int32_t* outputs,

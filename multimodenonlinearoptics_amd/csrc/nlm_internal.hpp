@@ -93,6 +93,10 @@ struct nlm_plan_s {
   hipGraphExec_t bigExec = nullptr;
   int bigKey[6] = {0, 0, 0, 0, 0, 0};
   const void* bigStatePtr = nullptr;
+  // Last asynchronous call that used the plan's scratch (bigState, the any-length path's table
+  // and workspaces): the next call on them may be on another stream (nlm_plan_set_stream).
+  hipEvent_t scratchDone = nullptr;
+  bool scratchBusy = false, scratchUsed = false;
   DevBuf<cplx> anyScratch;  // workspaces of the any-length path (nlm_any.hip) when they exceed LDS
   DevBuf<cplx> stepTab;  // RK4 step propagators of one-mode undepleted media [nZ][N][2]
   int stepTable = 1;      // use them (nlm_plan_set_step_table)
@@ -115,6 +119,11 @@ int launch_prop_kernel(nlm_plan_s* p, const KParams& kp);
 // uses_step_table(p)); allocates nothing
 int launch_prop_kernel_tab(nlm_plan_s* p, const KParams& kp, cplx* tab, bool may_tune = false);
 bool uses_step_table(const nlm_plan_s* p);
+// Before work on the plan's scratch: the stream waits for the asynchronous call that used it
+// last.  A capturing stream is left alone; the order of its replays is the caller's.
+int scratch_wait(nlm_plan_s* p);
+// After an asynchronous call: records it if it used the scratch.
+int scratch_mark(nlm_plan_s* p);
 int get_twiddles(int n, const cplx** out);
 // input channel feeding each mode (-1: none), src/_NonlinearMedium.hpp:164-198
 void input_channels(int nS, int nCh, int inputMode, int* inPos);
