@@ -433,10 +433,10 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
 extern "C" int nlm_multi_launch(nlm_multi* m) {
   if (!m) return set_err(NLM_INVALID_ARGUMENT, "null batch");
   if (!m->exec) return NLM_OK;
-  {
-    std::lock_guard<std::mutex> lk(m->outMu);
-    m->hostOutOf = false;
-  }
+  // held until the graph is queued: an output in between would keep the launch before's
+  // results as this one's
+  std::lock_guard<std::mutex> lk(m->outMu);
+  m->hostOutOf = false;
   HIP_TRY(hipEventRecord(m->t0, m->stream));
   HIP_TRY(hipGraphLaunch(m->exec, m->stream));
   HIP_TRY(hipEventRecord(m->t1, m->stream));
