@@ -213,11 +213,24 @@ typedef struct nlm_multi_s nlm_multi;
  * largest nFreqs first, a quarter of the device memory and half of what is free at
  * most; classes beyond that generate their pump rows in the kernel. */
 int nlm_multi_create(int n, const nlm_multi_item* items, int autotune, nlm_multi** out);
+/* The same with a limit of stage_bytes on that buffer: 0 stages nothing, below 0 is the
+ * rule above.  What is staged decides how a class's kernel runs (nlm_multi_form) and with
+ * it the last bits of its results, which by the rule above depend on the memory that is
+ * free at creation. */
+int nlm_multi_create_staged(int n, const nlm_multi_item* items, int autotune, int64_t stage_bytes, nlm_multi** out);
 int nlm_multi_launch(nlm_multi* batch);             /* one graph launch, asynchronous */
 int nlm_multi_sync(nlm_multi* batch, double* ms);   /* wait; ms = device time of the last launch */
 int nlm_multi_output(nlm_multi* batch, int i, double* out);  /* n_out*N complex of instance i */
 int nlm_multi_classes(nlm_multi* batch);
 int nlm_multi_grid(nlm_multi* batch, int c, int32_t* model, int32_t* log2n, int32_t* count, int32_t* grid);
+/* How the kernel of class c runs one instance, and the bytes staged for the class. */
+enum {
+  NLM_MULTI_FIELD = 0,   /* all modes in the same lanes, pump rows from the media's grids */
+  NLM_MULTI_INLINE = 1,  /* the same, the pump rows generated in the kernel */
+  NLM_MULTI_MODES = 2,   /* lanes of its own per mode, pump rows from grids or staged */
+  NLM_MULTI_TABLE = 3    /* one mode, with a staged step table */
+};
+int nlm_multi_form(nlm_multi* batch, int c, int32_t* form, int64_t* staged_bytes);
 int nlm_multi_destroy(nlm_multi* batch);
 
 /* Single-signal-mode undepleted media (Chi3, Chi2PDC): propagate with the

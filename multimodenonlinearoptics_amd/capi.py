@@ -18,7 +18,7 @@ SYMBOLS = [
     "nlm_plan_sync", "nlm_last_error", "nlm_version", "nlm_greens_forward", "nlm_greens_adjoint", "nlm_greens_forward_dev",
     "nlm_greens_adjoint_dev", "nlm_batch_forward_dev", "nlm_batch_adjoint_dev", "nlm_plan_owns_device_of",
     "nlm_multi_create", "nlm_multi_launch", "nlm_multi_sync", "nlm_multi_output", "nlm_multi_classes",
-    "nlm_multi_grid", "nlm_multi_destroy", "nlm_batch_forward", "nlm_batch_adjoint",
+    "nlm_multi_grid", "nlm_multi_create_staged", "nlm_multi_form", "nlm_multi_destroy", "nlm_batch_forward", "nlm_batch_adjoint",
     "nlm_greens_compose_dev", "nlm_greens_cascade", "nlm_pump_import",
     "nlm_batch_grids", "nlm_gaussian_covariance", "nlm_gram", "nlm_gemm_nt", "nlm_greens_noalloc",
     "nlm_fft_schedule",

@@ -1395,7 +1395,7 @@ Grid Cascade::batchSignalSimulation(const Grid& inputProfs, bool inTimeDomain, b
 // ---------------------------------------------------------------------------
 
 MultiBatch::MultiBatch(const std::vector<Medium*>& media, const std::vector<std::vector<cd>>& inputs,
-                       bool inTimeDomain, bool autotune, bool stageRows)
+                       bool inTimeDomain, bool autotune, bool stageRows, long long stageLimit)
     : media_(media) {
   if (media.size() != inputs.size()) throw std::invalid_argument("one input row per medium is required");
   const size_t n = media.size();
@@ -1434,7 +1434,7 @@ MultiBatch::MultiBatch(const std::vector<Medium*>& media, const std::vector<std:
     }
     outLen_.push_back(md->nS_ * md->N_);
   }
-  check(nlm_multi_create((int)n, items.data(), (autotune ? 1 : 0) | (stageRows ? 2 : 0), &m_));
+  check(nlm_multi_create_staged((int)n, items.data(), (autotune ? 1 : 0) | (stageRows ? 2 : 0), stageLimit, &m_));
 }
 
 MultiBatch::~MultiBatch() {
@@ -1463,6 +1463,18 @@ std::vector<std::array<int, 4>> MultiBatch::classes() const {
     int32_t model, l, count, grid;
     check(nlm_multi_grid(m_, c, &model, &l, &count, &grid));
     r.push_back({model, l, count, grid});
+  }
+  return r;
+}
+
+std::vector<std::pair<int, long long>> MultiBatch::forms() const {
+  std::vector<std::pair<int, long long>> r;
+  const int nc = nlm_multi_classes(m_);
+  for (int c = 0; c < nc; c++) {
+    int32_t form;
+    int64_t bytes;
+    check(nlm_multi_form(m_, c, &form, &bytes));
+    r.push_back({form, (long long)bytes});
   }
   return r;
 }

@@ -327,10 +327,10 @@ class Chi3GNLSE : public FullyNonlinearMedium {
 // runPump=True) of that medium (src/_NonlinearMedium.cpp:378-444).
 class MultiBatch {
  public:
-  // stageRows: nFreqs 4096 media with a generated pump stage their pump rows in a
-  // device buffer at the start of each launch (see nlm_multi_create)
+  // stageLimit: bytes of device memory that each launch may form step tables and pump rows in
+  // (0 none, below 0 the rule of nlm_multi_create); stageRows has no effect
   MultiBatch(const std::vector<Medium*>& media, const std::vector<std::vector<cd>>& inputs, bool inTimeDomain,
-             bool autotune, bool stageRows = false);
+             bool autotune, bool stageRows = false, long long stageLimit = -1);
   ~MultiBatch();
   MultiBatch(const MultiBatch&) = delete;
   MultiBatch& operator=(const MultiBatch&) = delete;
@@ -343,6 +343,7 @@ class MultiBatch {
   std::vector<cd> output(int i) const;
   int size() const { return (int)media_.size(); }
   std::vector<std::array<int, 4>> classes() const;  // (model, log2 N, instances, persistent workgroups)
+  std::vector<std::pair<int, long long>> forms() const;  // (NLM_MULTI_*, staged bytes) of each class
 
  private:
   std::vector<Medium*> media_;

@@ -64,6 +64,7 @@ struct MultiClass {
   int model, L, count, grid;
   int form;         // MULTI_FIELD, MULTI_INLINE, MULTI_MODES or MULTI_TAB
   int stage;        // STAGE_*: what is formed before the propagation kernel
+  size_t staged;    // its bytes
   int chunkOff = 0, nChunks = 0;
   multi_fn fn;
   size_t orderOff;  // offset of this class's instance order in the order array
@@ -132,6 +133,11 @@ extern "C" int nlm_multi_destroy(nlm_multi* m) {
 }
 
 extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune, nlm_multi** out) {
+  return nlm_multi_create_staged(n, items, autotune, -1, out);
+}
+
+extern "C" int nlm_multi_create_staged(int n, const nlm_multi_item* items, int autotune, int64_t stage_bytes,
+                                       nlm_multi** out) {
   if (!out || n < 0 || (n > 0 && !items)) return set_err(NLM_INVALID_ARGUMENT, "invalid arguments");
   *out = nullptr;
   autotune &= 1;  // bit 1 (stage the pump rows) is accepted; staging is the rule below
@@ -240,8 +246,8 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
     }
   }
   // What each class stages, the largest fields first (they are the longest chains and
-  // gain most) while everything staged fits a quarter of the device memory and half
-  // of what is free: the step table of one-mode media (32 bytes per point and step), or
+  // gain most) while everything staged fits the caller's limit, by default a quarter of the
+  // device memory and half of what is free: the step table of one-mode media (32 bytes per point and step), or
   // the pump rows of multi-mode media with a generated pump (as many bytes).  A class
   // that does not fit generates its rows in the kernel, or reads its grids.
   // SHG / PDC media of nFreqs 256..4096, nZSteps 200..4000, launch ms with every class
@@ -252,13 +258,14 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
   std::vector<std::vector<int>> members;
   size_t freeB = 0, totalB = 0;
   if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) freeB = totalB = 0;
-  size_t budget = std::min(totalB / 4, freeB / 2), stageTot = 0;
+  size_t budget = stage_bytes < 0 ? std::min(totalB / 4, freeB / 2) : (size_t)stage_bytes, stageTot = 0;
   for (auto& kv : byClass) {
     MultiClass c;
     c.model = std::get<0>(kv.first);
     c.L = std::get<1>(kv.first);
     const bool groups = pick_multi(c.model, c.L, MULTI_MODES) != nullptr;
     c.stage = STAGE_NONE;
+    c.staged = 0;
     c.form = std::get<2>(kv.first) ? MULTI_INLINE : groups ? MULTI_MODES : MULTI_FIELD;
     cls.push_back(c);
     members.push_back(kv.second);
@@ -275,6 +282,7 @@ extern "C" int nlm_multi_create(int n, const nlm_multi_item* items, int autotune
     if (need * sizeof(cplx) > budget) continue;
     budget -= need * sizeof(cplx);
     stageTot += need;
+    c.staged = need * sizeof(cplx);
     c.stage = !table ? STAGE_ROWS : inl ? STAGE_TAB : STAGE_TAB_GRID;
     c.form = table ? MULTI_TAB : MULTI_MODES;
   }
@@ -477,6 +485,14 @@ extern "C" int nlm_multi_grid(nlm_multi* m, int c, int32_t* model, int32_t* log2
   if (log2n) *log2n = m->classes[c].L;
   if (count) *count = m->classes[c].count;
   if (grid) *grid = m->classes[c].grid;
+  return NLM_OK;
+}
+
+extern "C" int nlm_multi_form(nlm_multi* m, int c, int32_t* form, int64_t* staged_bytes) {
+  if (!m) return set_err(NLM_INVALID_ARGUMENT, "null batch");
+  if (c < 0 || c >= (int)m->classes.size()) return set_err(NLM_INVALID_ARGUMENT, "class index out of range");
+  if (form) *form = m->classes[c].form;
+  if (staged_bytes) *staged_bytes = (int64_t)m->classes[c].staged;
   return NLM_OK;
 }
 

@@ -29,10 +29,10 @@ struct MultiInst {
 
 // How a class's kernel runs one instance per workgroup.
 enum {
-  MULTI_FIELD = 0,   // all modes in the same lanes, pump rows from a grid
-  MULTI_INLINE = 1,  // the same, the pump rows generated in the kernel
-  MULTI_MODES = 2,   // one lane group per mode (nlm_modes.hpp), pump rows from a grid
-  MULTI_TAB = 3,     // one mode with a step table
+  MULTI_FIELD = NLM_MULTI_FIELD,    // all modes in the same lanes, pump rows from a grid
+  MULTI_INLINE = NLM_MULTI_INLINE,  // the same, the pump rows generated in the kernel
+  MULTI_MODES = NLM_MULTI_MODES,    // one lane group per mode (nlm_modes.hpp), pump rows from a grid
+  MULTI_TAB = NLM_MULTI_TABLE,      // one mode with a step table
 };
 
 template <class M, int L, int FORM>

@@ -417,15 +417,15 @@ PYBIND11_MODULE(nonlinearmedium, m) {
                               "propagated together by one graph launch (extension).  output(i) equals "
                               "media[i].batchSignalSimulation(inputs[i][None], inTimeDomain)[0].")
       .def(py::init([](const py::list& media, const py::list& inputs, bool inTimeDomain, bool autotune,
-                       bool stagePumpRows) {
+                       bool stagePumpRows, long long stageLimit) {
              std::vector<Medium*> v;
              for (auto h : media) v.push_back(&h.cast<Medium&>());
              std::vector<std::vector<cd>> in;
              for (auto h : inputs) in.push_back(to_vec(h.cast<carr>()));
-             return new nlm::MultiBatch(v, in, inTimeDomain, autotune, stagePumpRows);
+             return new nlm::MultiBatch(v, in, inTimeDomain, autotune, stagePumpRows, stageLimit);
            }),
            "media"_a, "inputs"_a, "inTimeDomain"_a = false, "autotune"_a = true, "stagePumpRows"_a = false,
-           py::keep_alive<1, 2>())
+           "stageLimit"_a = -1, py::keep_alive<1, 2>())
       .def("launch", [](nlm::MultiBatch& b) {
         py::gil_scoped_release nogil;
         b.launch();
@@ -446,7 +446,14 @@ PYBIND11_MODULE(nonlinearmedium, m) {
       }, "i"_a)
       .def("__len__", &nlm::MultiBatch::size)
       .def("classes", &nlm::MultiBatch::classes,
-           "(model id, log2 nFreqs, instances, persistent workgroups) of each kernel class");
+           "(model id, log2 nFreqs, instances, persistent workgroups) of each kernel class")
+      .def("forms", [](const nlm::MultiBatch& b) {
+        static const char* const names[] = {"field", "inline", "modes", "table"};
+        std::vector<std::pair<std::string, long long>> r;
+        for (const auto& f : b.forms()) r.emplace_back(names[f.first], f.second);
+        return r;
+      }, "(form, staged bytes) of each kernel class: 'table' and 'modes' media with staged bytes read what each "
+         "launch forms up front, 'inline' ones generate their pump rows in the kernel");
 
   // Cascade, src/nlmModulePy.cpp:170-211
   cascade.def(py::init([](const py::list& media, const std::vector<std::map<unsigned, unsigned>>& conns, bool share) {
