@@ -254,43 +254,56 @@ extern "C" int nlm_multi_create_staged(int n, const nlm_multi_item* items, int a
   // generating its rows and the modes sharing lanes -> now: 2000 media 156 -> 132 (the
   // N = 4096 tables take 54 GB of the budget, the other classes generate theirs), 500
   // media 149 -> 68 (all staged, 27 GB).
+  // Where the buffer cannot be had after all (memory taken since by another thread or process),
+  // half of it is tried, and in the end none.
   std::vector<MultiClass> cls;
   std::vector<std::vector<int>> members;
-  size_t freeB = 0, totalB = 0;
-  if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) freeB = totalB = 0;
-  size_t budget = stage_bytes < 0 ? std::min(totalB / 4, freeB / 2) : (size_t)stage_bytes, stageTot = 0;
   for (auto& kv : byClass) {
     MultiClass c;
     c.model = std::get<0>(kv.first);
     c.L = std::get<1>(kv.first);
-    const bool groups = pick_multi(c.model, c.L, MULTI_MODES) != nullptr;
-    c.stage = STAGE_NONE;
-    c.staged = 0;
-    c.form = std::get<2>(kv.first) ? MULTI_INLINE : groups ? MULTI_MODES : MULTI_FIELD;
     cls.push_back(c);
     members.push_back(kv.second);
   }
   std::vector<int> bySize(cls.size());
   for (size_t k = 0; k < cls.size(); k++) bySize[k] = (int)k;
   std::stable_sort(bySize.begin(), bySize.end(), [&](int a, int b) { return cls[a].L > cls[b].L; });
-  for (int k : bySize) {
-    MultiClass& c = cls[k];
-    const bool inl = c.form == MULTI_INLINE, table = pick_multi(c.model, c.L, MULTI_TAB) != nullptr;
-    if (!table && !(inl && pick_multi(c.model, c.L, MULTI_MODES))) continue;
-    size_t need = 0;
-    for (int i : members[k]) need += (size_t)2 * hi[i].nZ * m->N[i];
-    if (need * sizeof(cplx) > budget) continue;
-    budget -= need * sizeof(cplx);
-    stageTot += need;
-    c.staged = need * sizeof(cplx);
-    c.stage = !table ? STAGE_ROWS : inl ? STAGE_TAB : STAGE_TAB_GRID;
-    c.form = table ? MULTI_TAB : MULTI_MODES;
+  // the forms for a budget in bytes; returns the elements that they stage
+  const auto choose = [&](size_t budget) {
+    size_t total = 0;
+    for (int k : bySize) {
+      MultiClass& c = cls[k];
+      const nlm_multi_item& it = items[members[k][0]];
+      const bool inl = it.plan->nP > 0 && it.envelope != nullptr;
+      const bool groups = pick_multi(c.model, c.L, MULTI_MODES) != nullptr;
+      const bool table = pick_multi(c.model, c.L, MULTI_TAB) != nullptr;
+      c.stage = STAGE_NONE;
+      c.staged = 0;
+      c.form = inl ? MULTI_INLINE : groups ? MULTI_MODES : MULTI_FIELD;
+      if (!table && !(inl && groups)) continue;
+      size_t need = 0;
+      for (int i : members[k]) need += (size_t)2 * hi[i].nZ * m->N[i];
+      if (need * sizeof(cplx) > budget) continue;
+      budget -= need * sizeof(cplx);
+      total += need;
+      c.staged = need * sizeof(cplx);
+      c.stage = !table ? STAGE_ROWS : inl ? STAGE_TAB : STAGE_TAB_GRID;
+      c.form = table ? MULTI_TAB : MULTI_MODES;
+    }
+    return total;
+  };
+  size_t freeB = 0, totalB = 0;
+  if (hipMemGetInfo(&freeB, &totalB) != hipSuccess) freeB = totalB = 0;
+  size_t stageTot = choose(stage_bytes < 0 ? std::min(totalB / 4, freeB / 2) : (size_t)stage_bytes);
+  while (m->stageBuf.ensure(stageTot)) {
+    (void)hipGetLastError();
+    stageTot = choose(stageTot * sizeof(cplx) / 2);
   }
   for (auto& c : cls) {
     c.fn = pick_multi(c.model, c.L, c.form);
     if (!c.fn) return fail(set_err(NLM_INVALID_ARGUMENT, "heterogeneous batches take nFreqs a power of two, 32..4096"));
   }
-  if ((e = m->counters.ensure(cls.size() + 1)) || (e = m->stageBuf.ensure(stageTot))) return fail(e);
+  if ((e = m->counters.ensure(cls.size() + 1))) return fail(e);
   std::vector<int> hchunks;
   size_t stageOff = 0;
   // the classes' longest-first orders

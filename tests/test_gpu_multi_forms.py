@@ -70,3 +70,23 @@ def test_limit_holds_the_largest_class(nlm, oracle):
     assert f == {(1, 1024): ("table", need), (1, 256): ("inline", 0)}
     f = forms(batch(nlm, oracle, cases, stageLimit=need - 1))
     assert f[(1, 1024)] == ("inline", 0)
+
+
+def test_staging_that_cannot_be_had(nlm):
+    """More than the card has: the largest class falls back to generated rows, the small one is
+    staged within what is left, and the results are those of that choice made at once."""
+    N, nZ = 4096, 20000
+    small = dict(relativeLength=1.0, nlLength=1.0, beta2=0.1, beta2s=-0.2, tMax=20, tPrecision=256, nZSteps=50)
+    big = dict(small, tPrecision=N, nZSteps=nZ)
+    count = 400 * 10 ** 9 // (2 * nZ * N * 16)
+    media = [nlm.Chi2PDC(**big) for _ in range(count)] + [nlm.Chi2PDC(**small)]
+    r = np.random.default_rng(0)
+    xs = [r.standard_normal(m.omega.size) + 0j for m in media]
+    got = []
+    for limit in (1 << 60, 1 << 30):
+        b = nlm.MultiBatch(media, xs, inTimeDomain=True, autotune=False, stageLimit=limit)
+        assert forms(b) == {(1, N): ("inline", 0), (1, 256): ("table", 2 * 50 * 256 * 16)}
+        print("created, limit", limit, "ms", b.run(), flush=True)
+        got.append([b.output(i) for i in (0, count - 1, count)])
+    for a, c in zip(*got):
+        assert np.isfinite(a).all() and np.array_equal(a, c)
