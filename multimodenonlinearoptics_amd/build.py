@@ -57,22 +57,22 @@ def build(force=False, jobs=None, verbose=False):
     objs = []
     o = os.path.join(OBJ, "nlm_device.o")
     objs.append(o)
-    deps = _deps("nlm_device.hip", "nlm_internal.hpp", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
+    deps = _deps("nlm_device.hip", "nlm_internal.hpp", "nlm_copy.hpp", "nlm_tab.hpp", "nlm_quad.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_device.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_adjoint.o")
     objs.append(o)
-    deps = _deps("nlm_adjoint.hip", "nlm_adjoint.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_adjoint.hip", "nlm_adjoint.hpp", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_adjoint.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_big.o")
     objs.append(o)
-    deps = _deps("nlm_big.hip", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_big.hip", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_big.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_multi.o")
     objs.append(o)
-    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_quad.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_multi.hip", "nlm_multi.hpp", "nlm_modes.hpp", "nlm_tab.hpp", "nlm_quad.hpp", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_multi_stage.o")
@@ -82,22 +82,22 @@ def build(force=False, jobs=None, verbose=False):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_multi_stage.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_compose.o")
     objs.append(o)
-    deps = _deps("nlm_compose.hip", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_compose.hip", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_compose.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_any.o")
     objs.append(o)
-    deps = _deps("nlm_any.hip", "nlm_mix.hpp", "nlm_modes.hpp", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_any.hip", "nlm_mix.hpp", "nlm_modes.hpp", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_any.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_copy.o")
     objs.append(o)
-    deps = _deps("nlm_copy.hip", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_copy.hip", "nlm_copy.hpp")
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_copy.hip"), "-o", o])
     o = os.path.join(OBJ, "nlm_noalloc.o")
     objs.append(o)
-    deps = _deps("nlm_noalloc.hip", "nlm_internal.hpp", *dev_hdrs)
+    deps = _deps("nlm_noalloc.hip", "nlm_internal.hpp", "nlm_copy.hpp", *dev_hdrs)
     if force or _stale(o, deps):
         steps.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(CSRC, "nlm_noalloc.hip"), "-o", o])
     for v in range(4):  # FFT schedule variants of the step-table kernel (chosen by the autotuner)

@@ -14,12 +14,16 @@
 #include <sys/types.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <condition_variable>
 #include <cstring>
 #include <functional>
+#include <mutex>
 #include <thread>
+#include <vector>
 
-#include "nlm_internal.hpp"
+#include "../../include/nlm.h"
+#include "nlm_copy.hpp"
 
 namespace {
 
@@ -107,14 +111,14 @@ class Helpers {
 
  private:
   bool start() {
-    if (pid_ == getpid()) return true;
-    if (pid_ != 0) return false;  // a forked child has none of its parent's threads
+    if (started_ > 0 && pid_ != getpid()) return false;  // a forked child has none of its parent's threads
+    pid_ = getpid();
+    // each part once: helpers that could not be started are started by a later copy
     try {
-      for (int k = 1; k <= HELPERS; k++) std::thread([this, k] { loop(k); }).detach();
+      for (; started_ < HELPERS; started_++) std::thread([this, k = started_ + 1] { loop(k); }).detach();
     } catch (...) {
       return false;
     }
-    pid_ = getpid();
     return true;
   }
   void loop(int part) {
@@ -140,6 +144,7 @@ class Helpers {
   const std::function<void(int)>* body_ = nullptr;
   int left_ = 0;
   unsigned long round_ = 0;
+  int started_ = 0;
   pid_t pid_ = 0;
 };
 
@@ -243,15 +248,3 @@ int nlm_to_device(void* dev, const void* host, size_t bytes, hipStream_t s) {
   const hipError_t e = hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s);
   return e == hipSuccess ? NLM_OK : failed(e);
 }
-
-bool nlm_on_device(const void* ptr, int device) {
-  if (!ptr) return false;
-  hipPointerAttribute_t a;
-  if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
-  return a.type == hipMemoryTypeDevice && a.device == device;
-}
-
-extern "C" int nlm_plan_owns_device_of(nlm_plan* p, const void* ptr) { return p && nlm_on_device(ptr, p->device) ? 1 : 0; }

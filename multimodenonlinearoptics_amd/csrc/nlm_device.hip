@@ -418,6 +418,18 @@ extern "C" int nlm_model_ncoef(int model, int32_t* nc, int32_t* ncc, int32_t* ns
   return NLM_OK;
 }
 
+bool nlm_on_device(const void* ptr, int device) {
+  if (!ptr) return false;
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, ptr) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice && a.device == device;
+}
+
+extern "C" int nlm_plan_owns_device_of(nlm_plan* p, const void* ptr) { return p && nlm_on_device(ptr, p->device) ? 1 : 0; }
+
 static int upload(DevBuf<cplx>& b, const double* src, size_t count, hipStream_t s) {
   int e = b.ensure(count);
   if (e) return e;

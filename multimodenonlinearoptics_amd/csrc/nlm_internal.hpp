@@ -9,9 +9,8 @@
 #include <vector>
 
 #include "../../include/nlm.h"
+#include "nlm_copy.hpp"
 #include "nlm_prop.hpp"
-
-int set_err(int kind, const std::string& msg);
 
 #define HIP_TRY(expr)                                                                              \
   do {                                                                                             \
@@ -46,16 +45,6 @@ struct DevBuf {
   }
 };
 
-// Copies to and from a caller's pageable memory (nlm_copy.hip).  nlm_to_host returns
-// when every item is in place (items with a null host pointer are skipped) and the
-// stream's work before it is done; nlm_to_device when `host` may be reused.
-struct HostCopy {
-  void* host;
-  const void* dev;
-  size_t bytes;
-};
-int nlm_to_host(const HostCopy* items, int n, hipStream_t s);
-int nlm_to_device(void* dev, const void* host, size_t bytes, hipStream_t s);
 // whether ptr is memory of `device` that this process's HIP runtime knows
 bool nlm_on_device(const void* ptr, int device);
 

@@ -1,0 +1,36 @@
+"""The logic of the device-to-host copies (nlm_copy.hip) on a CPU: the file is compiled with g++
+over a small runtime whose device memory is host memory (fake_hip/), and each scenario of
+copy_host_driver.cpp is run in a process of its own."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+
+
+@pytest.fixture(scope="module")
+def driver(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("copies") / "driver")
+    r = subprocess.run(["g++", "-O1", "-g", "-std=c++17", "-Wall", "-I" + os.path.join(HERE, "fake_hip"),
+                        "-I" + os.path.join(HERE, "..", "include"), os.path.join(HERE, "copy_host_driver.cpp"),
+                        "-o", exe, "-lpthread", "-ldl"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout
+    return exe
+
+
+def run(driver, scenario):
+    r = subprocess.run([driver, scenario], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
+def test_every_size_arrives(driver):
+    run(driver, "sizes")
+
+
+def test_helpers_that_start_late(driver):
+    """A helper thread that cannot be started is started by a later copy, the others not again."""
+    run(driver, "helpers")
