@@ -17,10 +17,9 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
-#include <functional>
 #include <mutex>
+#include <new>
 #include <thread>
-#include <vector>
 
 #include "../../include/nlm.h"
 #include "nlm_copy.hpp"
@@ -49,7 +48,8 @@ struct Staging {
 // Staging areas: taken for the length of one copy, so concurrent callers never share
 // one; at most MAX_IDLE are kept, the others are freed when they come back.
 std::mutex g_mu;
-std::vector<Staging*> g_idle;
+Staging* g_idle[MAX_IDLE];
+int g_idles = 0;
 
 hipError_t take(Staging** out) {
   int dev = 0;
@@ -57,14 +57,15 @@ hipError_t take(Staging** out) {
   if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    for (size_t k = 0; k < g_idle.size(); k++)
+    for (int k = 0; k < g_idles; k++)
       if (g_idle[k]->device == dev) {
         *out = g_idle[k];
-        g_idle.erase(g_idle.begin() + (long)k);
+        g_idle[k] = g_idle[--g_idles];
         return hipSuccess;
       }
   }
-  Staging* s = new Staging();
+  Staging* s = new (std::nothrow) Staging();
+  if (!s) return hipErrorOutOfMemory;
   s->device = dev;
   e = hipHostMalloc((void**)&s->buf, SLOTS * PIECE, hipHostMallocDefault);
   for (int k = 0; k < SLOTS && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming);
@@ -79,33 +80,38 @@ hipError_t take(Staging** out) {
 void give(Staging* s) {
   {
     std::lock_guard<std::mutex> lk(g_mu);
-    if ((int)g_idle.size() < MAX_IDLE) {
-      g_idle.push_back(s);
+    if (g_idles < MAX_IDLE) {
+      g_idle[g_idles++] = s;
       return;
     }
   }
   s->destroy();
 }
 
+// Work for the caller and the helpers: part 0..PARTS-1 of it on each.
+struct Job {
+  virtual void run(int part) = 0;
+};
+
 // Helper threads, started at the first large copy and kept for the process.  One copy
 // uses them at a time; another that comes meanwhile does without.
 class Helpers {
  public:
-  // body(part) for part = 0..PARTS-1 on the caller and the helpers; false if they are busy
-  bool run(const std::function<void(int)>& body) {
+  // every part of the job; false if the helpers are busy
+  bool run(Job& job) {
     std::unique_lock<std::mutex> use(use_, std::try_to_lock);
     if (!use.owns_lock() || !start()) return false;
     {
       std::lock_guard<std::mutex> lk(mu_);
-      body_ = &body;
+      job_ = &job;
       left_ = HELPERS;
       round_++;
     }
     go_.notify_all();
-    body(0);
+    job.run(0);
     std::unique_lock<std::mutex> lk(mu_);
     done_.wait(lk, [&] { return left_ == 0; });
-    body_ = nullptr;
+    job_ = nullptr;
     return true;
   }
 
@@ -124,14 +130,14 @@ class Helpers {
   void loop(int part) {
     unsigned long seen = 0;
     for (;;) {
-      const std::function<void(int)>* body;
+      Job* job;
       {
         std::unique_lock<std::mutex> lk(mu_);
         go_.wait(lk, [&] { return round_ != seen; });
         seen = round_;
-        body = body_;
+        job = job_;
       }
-      (*body)(part);
+      job->run(part);
       {
         std::lock_guard<std::mutex> lk(mu_);
         left_--;
@@ -141,7 +147,7 @@ class Helpers {
   }
   std::mutex use_, mu_;
   std::condition_variable go_, done_;
-  const std::function<void(int)>* body_ = nullptr;
+  Job* job_ = nullptr;
   int left_ = 0;
   unsigned long round_ = 0;
   int started_ = 0;
@@ -179,19 +185,40 @@ hipError_t share(Staging* st, char* host, const char* dev, size_t bytes, int par
 }
 
 hipError_t large(Staging* st, char* host, const char* dev, size_t bytes, hipStream_t s) {
-  hipError_t errs[PARTS] = {};
-  const int device = st->device;
-  const std::function<void(int)> body = [&](int part) {
-    if (part > 0) {
-      errs[part] = hipSetDevice(device);
-      if (errs[part] != hipSuccess) return;
+  struct Shares : Job {
+    Staging* st;
+    char* host;
+    const char* dev;
+    size_t bytes;
+    hipStream_t s;
+    hipError_t errs[PARTS] = {};
+    void run(int part) override {
+      if (part > 0) {
+        errs[part] = hipSetDevice(st->device);
+        if (errs[part] != hipSuccess) return;
+      }
+      errs[part] = share(st, host, dev, bytes, part, PARTS, s);
     }
-    errs[part] = share(st, host, dev, bytes, part, PARTS, s);
-  };
-  if (!helpers().run(body)) return share(st, host, dev, bytes, 0, 1, s);
-  for (hipError_t e : errs)
+  } job;
+  job.st = st;
+  job.host = host;
+  job.dev = dev;
+  job.bytes = bytes;
+  job.s = s;
+  if (!helpers().run(job)) return share(st, host, dev, bytes, 0, 1, s);
+  for (hipError_t e : job.errs)
     if (e != hipSuccess) return e;
   return hipSuccess;
+}
+
+// Without a staging area (no pinned memory left): the runtime's own copies.
+hipError_t plain(const HostCopy* items, int n, hipStream_t s) {
+  hipError_t e = hipSuccess;
+  for (int i = 0; i < n && e == hipSuccess; i++)
+    if (items[i].host && items[i].bytes)
+      e = hipMemcpyAsync(items[i].host, items[i].dev, items[i].bytes, hipMemcpyDeviceToHost, s);
+  const hipError_t w = hipStreamSynchronize(s);
+  return e == hipSuccess ? w : e;
 }
 
 int failed(hipError_t e) {
@@ -203,7 +230,11 @@ int failed(hipError_t e) {
 int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
   Staging* st = nullptr;
   hipError_t e = take(&st);
-  if (e != hipSuccess) return failed(e);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    e = plain(items, n, s);
+    return e == hipSuccess ? NLM_OK : failed(e);
+  }
   size_t at = 0;
   int first = 0;
   // small items are gathered in the staging area and waited for together

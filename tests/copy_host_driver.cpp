@@ -4,6 +4,7 @@
 #include <pthread.h>
 
 #include <cstdio>
+#include <vector>
 
 #include "../multimodenonlinearoptics_amd/csrc/nlm_copy.hip"
 
@@ -63,6 +64,16 @@ int main(int argc, char** argv) {
     threadsAllowed = 1 << 30;
     for (unsigned r = 0; r < 20; r++) copy({13 * MB + r}, &s, r);
     CHECK(threadsMade == 3);
+  } else if (what == "no area") {
+    fake::failHostMalloc = true;
+    copy({100, MB, 5 * MB}, &s, 0);
+    fake::failHostMalloc = false;
+    fake::failEventCreate = true;
+    copy({100, MB, 5 * MB}, &s, 1);
+    CHECK(fake::areas == 0 && fake::events == 0 && hipGetLastError() == hipSuccess);
+    fake::failEventCreate = false;
+    copy({100, MB, 5 * MB}, &s, 2);
+    CHECK(fake::areas == 1);
   } else {
     std::printf("unknown scenario\n");
     return 2;

@@ -34,3 +34,8 @@ def test_every_size_arrives(driver):
 def test_helpers_that_start_late(driver):
     """A helper thread that cannot be started is started by a later copy, the others not again."""
     run(driver, "helpers")
+
+
+def test_no_pinned_memory(driver):
+    """Where no staging area can be allocated the copies are the runtime's own, with no error left."""
+    run(driver, "no area")
