@@ -51,9 +51,11 @@ std::mutex g_mu;
 Staging* g_idle[MAX_IDLE];
 int g_idles = 0;
 
-hipError_t take(Staging** out) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+// Of the stream's device, whichever is current: an event is recorded on its own device only.
+hipError_t take(hipStream_t stream, Staging** out) {
+  int dev = 0, cur = 0;
+  hipError_t e = hipStreamGetDevice(stream, &dev);
+  if (e == hipSuccess) e = hipGetDevice(&cur);
   if (e != hipSuccess) return e;
   {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -67,8 +69,10 @@ hipError_t take(Staging** out) {
   Staging* s = new (std::nothrow) Staging();
   if (!s) return hipErrorOutOfMemory;
   s->device = dev;
-  e = hipHostMalloc((void**)&s->buf, SLOTS * PIECE, hipHostMallocDefault);
+  if (cur != dev) e = hipSetDevice(dev);
+  if (e == hipSuccess) e = hipHostMalloc((void**)&s->buf, SLOTS * PIECE, hipHostMallocDefault);
   for (int k = 0; k < SLOTS && e == hipSuccess; k++) e = hipEventCreateWithFlags(&s->ev[k], hipEventDisableTiming);
+  if (cur != dev) (void)hipSetDevice(cur);
   if (e != hipSuccess) {
     s->destroy();
     return e;
@@ -229,7 +233,7 @@ int failed(hipError_t e) {
 
 int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
   Staging* st = nullptr;
-  hipError_t e = take(&st);
+  hipError_t e = take(s, &st);
   if (e != hipSuccess) {
     (void)hipGetLastError();
     e = plain(items, n, s);

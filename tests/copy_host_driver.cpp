@@ -74,6 +74,14 @@ int main(int argc, char** argv) {
     fake::failEventCreate = false;
     copy({100, MB, 5 * MB}, &s, 2);
     CHECK(fake::areas == 1);
+  } else if (what == "device") {
+    FakeStream other{1};
+    for (unsigned r = 0; r < 2; r++) {
+      copy({100, 5 * MB}, &other, r);
+      CHECK(fake::device == 0);
+      copy({100, 5 * MB}, &s, r);
+    }
+    CHECK(fake::areas == 2);
   } else {
     std::printf("unknown scenario\n");
     return 2;

@@ -39,3 +39,8 @@ def test_helpers_that_start_late(driver):
 def test_no_pinned_memory(driver):
     """Where no staging area can be allocated the copies are the runtime's own, with no error left."""
     run(driver, "no area")
+
+
+def test_stream_of_another_device(driver):
+    """A plan's results while another device is the current one, which stays so."""
+    run(driver, "device")
