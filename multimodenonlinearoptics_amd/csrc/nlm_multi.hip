@@ -24,6 +24,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <tuple>
 #include <vector>
 
@@ -482,7 +483,12 @@ extern "C" int nlm_multi_output(nlm_multi* m, int i, double* out) {
   std::lock_guard<std::mutex> lk(m->outMu);
   if (!m->hostOutOf) {
     const size_t total = m->outOff[m->n - 1] + (size_t)m->nOut[m->n - 1] * m->N[m->n - 1];
-    m->hostOut.resize(total);
+    try {
+      m->hostOut.resize(total);
+    } catch (const std::bad_alloc&) {  // no room on the host for all of them: this one alone
+      const HostCopy c = {out, m->outBuf.p + m->outOff[i], sizeof(cplx) * m->nOut[i] * m->N[i]};
+      return nlm_to_host(&c, 1, m->stream);
+    }
     const HostCopy c = {m->hostOut.data(), m->outBuf.p, total * sizeof(cplx)};
     if (int e = nlm_to_host(&c, 1, m->stream)) return e;
     m->hostOutOf = true;
