@@ -530,26 +530,39 @@ any_prop_fn pick_any_prop(int model) {
 
 bool nlm_any_size(int n) { return n >= 2 && n % 2 == 0 && (n < 8 || n > 8192 || (n & (n - 1)) != 0); }
 
-int nlm_any_prop(nlm_plan_s* p, const KParams& kp, bool may_alloc) {
+static bool one_mode(const nlm_plan_s* p) { return p->model == NLM_CHI3 || p->model == NLM_CHI2PDC; }
+
+bool nlm_any_uses_table(const nlm_plan_s* p, int fields) {
+  MixPlan mp;
+  return one_mode(p) && p->stepTable && mix_plan(p->N, p->nS, fields, false, &mp);
+}
+
+int nlm_any_prop(nlm_plan_s* p, const KParams& kp, cplx* tab, bool may_alloc) {
   const any_prop_fn fn = pick_any_prop(p->model);
   if (!fn) return set_err(NLM_INVALID_ARGUMENT, "unsupported model");
   if (kp.nFields <= 0) return NLM_OK;
   MixPlan mp;
-  const bool oneMode = p->model == NLM_CHI3 || p->model == NLM_CHI2PDC;
+  const bool oneMode = one_mode(p);
   // the one-mode media's mixed-radix kernel applies the step table, which needs a
-  // device buffer
-  if ((!oneMode || (p->stepTable && may_alloc)) &&
-      mix_plan(p->N, p->nS, kp.nFields, p->model == NLM_CHI3GNLSE, &mp)) {
+  // device buffer: the caller's, or the plan's, which a first call under stream capture
+  // cannot allocate (the general kernel then runs)
+  if (oneMode && !tab && may_alloc && nlm_any_uses_table(p, kp.nFields)) {
+    const size_t need = (size_t)p->nZ * p->N * 2;
+    if (p->stepTab.n >= need || !stream_capturing(p->stream)) {
+      if (int e = scratch_wait(p)) return e;
+      if (int e = p->stepTab.ensure(need)) return e;
+      tab = p->stepTab.p;
+    }
+  }
+  if ((!oneMode || tab) && mix_plan(p->N, p->nS, kp.nFields, p->model == NLM_CHI3GNLSE, &mp)) {
     const mix_fn mf = pick_mix(p->model, mp.R);
     if (!mf) return set_err(NLM_INVALID_ARGUMENT, "unsupported model / size");
     if (int e = get_twiddles(p->N, &mp.tw)) return e;
     KParams kq = kp;
     if (oneMode) {
-      if (int e = scratch_wait(p)) return e;
-      if (int e = p->stepTab.ensure((size_t)p->nZ * p->N * 2)) return e;
-      nlm_launch_step_table(p->model, p->coef.p, p->cconst.p, p->pumpT[0].p, p->N, p->nZ, p->stepTab.p, p->stream);
+      nlm_launch_step_table(p->model, p->coef.p, p->cconst.p, p->pumpT[0].p, p->N, p->nZ, tab, p->stream);
       HIP_TRY(hipGetLastError());
-      kq.tab = p->stepTab.p;
+      kq.tab = tab;
     }
     mf(kq, mp, (kp.nFields + mp.FPB - 1) / mp.FPB, p->stream);
     HIP_TRY(hipGetLastError());

@@ -712,8 +712,7 @@ bool nlm_big_supported(int model, int L) { return model == NLM_CHI3GNLSE && (L =
 bool nlm_big_better(nlm_plan* p, int rows) {
   constexpr int CUS = 256;
   if (p->model != NLM_CHI3GNLSE || p->L != 13 || p->nZ < 2 || rows > CUS) return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(p->stream, &st) != hipSuccess || st != hipStreamCaptureStatusNone) return false;
+  if (stream_capturing(p->stream)) return false;
   if (ensure_state(p, rows) == NLM_OK) return true;
   (void)hipGetLastError();
   return false;
@@ -762,9 +761,7 @@ int nlm_big_batch(nlm_plan* p, const cplx* in, int rows, int cols, int inTime, i
       p->bigKey[3] != inPos || p->bigKey[4] != nOut || p->bigKey[5] != outPos || p->bigStatePtr != p->bigState.p) {
     if (p->bigExec) {
       // an asynchronous call before this one may still be replaying it
-      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing(p->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)
-        HIP_TRY(hipStreamSynchronize(p->stream));
+      if (!stream_capturing(p->stream)) HIP_TRY(hipStreamSynchronize(p->stream));
       (void)hipGraphExecDestroy(p->bigExec);
     }
     p->bigExec = nullptr;

@@ -836,7 +836,7 @@ int tune_variant(nlm_plan* p, const KParams& kp, int grid, int* best) {
 }  // namespace
 
 int launch_prop_kernel_tab(nlm_plan* p, const KParams& kp0, cplx* tab, bool may_tune) {
-  if (p->L == 0) return nlm_any_prop(p, kp0, false);
+  if (p->L == 0) return nlm_any_prop(p, kp0, tab, false);
   if (p->L > 13)
     return set_err(NLM_INVALID_ARGUMENT, "nFreqs above 8192 is available for Chi3GNLSE batchSignalSimulation only");
   KParams kp = kp0;
@@ -969,13 +969,13 @@ extern "C" int nlm_grid_download(nlm_plan* p, int mode, double* sf, double* st) 
   return nlm_to_host(out, 2, p->stream);
 }
 
-static bool capturing(hipStream_t s) {
+bool stream_capturing(hipStream_t s) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(s, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
 }
 
 int scratch_wait(nlm_plan* p) {
-  if (capturing(p->stream)) return NLM_OK;
+  if (stream_capturing(p->stream)) return NLM_OK;
   p->scratchUsed = true;
   if (p->scratchBusy) HIP_TRY(hipStreamWaitEvent(p->stream, p->scratchDone, 0));
   return NLM_OK;

@@ -110,6 +110,7 @@ int launch_prop_kernel_tab(nlm_plan_s* p, const KParams& kp, cplx* tab, bool may
 bool uses_step_table(const nlm_plan_s* p);
 // Before work on the plan's scratch: the stream waits for the asynchronous call that used it
 // last.  A capturing stream is left alone; the order of its replays is the caller's.
+bool stream_capturing(hipStream_t s);
 int scratch_wait(nlm_plan_s* p);
 // After an asynchronous call: records it if it used the scratch.
 int scratch_mark(nlm_plan_s* p);
@@ -126,8 +127,11 @@ int nlm_big_batch(nlm_plan_s* p, const cplx* in, int rows, int cols, int inTime,
 // two, 2 and 4, or above 8192.  Plans of these lengths have L = 0.
 bool nlm_any_size(int n);
 // may_alloc = false: fail instead of allocating the device workspace that
-// lengths above the LDS workspace need
-int nlm_any_prop(nlm_plan_s* p, const KParams& kp, bool may_alloc = true);
+// lengths above the LDS workspace need.  tab: a step table [nZ][N][2] of the caller's
+// for the media that use one, or nullptr
+int nlm_any_prop(nlm_plan_s* p, const KParams& kp, cplx* tab = nullptr, bool may_alloc = true);
+// whether that many fields run with a step table where there is room for one
+bool nlm_any_uses_table(const nlm_plan_s* p, int fields);
 int nlm_any_pump_linear(nlm_plan_s* p, const double* strength_dev, double dzp);
 int nlm_any_pump_chi3(nlm_plan_s* p, double dzp);
 int nlm_any_pump_import(nlm_plan_s* p, int q, const cplx* sigF, int nzs, double dzs, const double* Ds,
