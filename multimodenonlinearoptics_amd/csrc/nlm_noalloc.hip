@@ -60,9 +60,13 @@ extern "C" int nlm_greens_noalloc(nlm_plan* p, int in_time, int n_in, const int3
   const int N = p->N;
   const size_t W = (size_t)n_out * N, nF = 2 * (size_t)n_in * N;
   const size_t gElems = nF * W;
-  const size_t tElems = uses_step_table(p) ? (size_t)p->nZ * N * 2 : 0;
+  size_t tElems = uses_step_table(p) ? (size_t)p->nZ * N * 2 : 0;
   // the table starts on a 256-byte boundary after G
   const size_t tOff = (gElems + 15) / 16 * 16;
+  // lengths that are not powers of two can do without one (in another kernel, slower and with
+  // other rounding than nlm_greens)
+  if (p->L == 0 && nlm_any_uses_table(p, (int)nF) && tOff + (size_t)p->nZ * N * 2 <= kScratchElems)
+    tElems = (size_t)p->nZ * N * 2;
   if (tOff + tElems > kScratchElems)
     return set_err(NLM_INVALID_ARGUMENT,
                    "nlm_greens_noalloc: the Green's rows (" + std::to_string(gElems * sizeof(cplx) >> 20) +
