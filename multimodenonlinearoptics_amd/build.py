@@ -52,7 +52,7 @@ def _run(cmd):
 
 def build(force=False, jobs=None, verbose=False):
     os.makedirs(OBJ, exist_ok=True)
-    dev_hdrs = ["nlm_fft.hpp", "nlm_models.hpp", "nlm_prop.hpp"]
+    dev_hdrs = ["nlm_fft.hpp", "nlm_sincos.hpp", "nlm_models.hpp", "nlm_prop.hpp"]
     steps = []
     objs = []
     o = os.path.join(OBJ, "nlm_device.o")

@@ -22,6 +22,8 @@
 #include <type_traits>
 #include <hip/hip_runtime.h>
 
+#include "nlm_sincos.hpp"
+
 struct __align__(16) cplx {
   double re, im;
 };
@@ -107,30 +109,6 @@ __device__ __forceinline__ void sincos_reduced(double a, double* s, double* c) {
     case 2: *s = -sr; *c = -cr; break;
     default: *s = -cr; *c = sr; break;
   }
-}
-
-// sin and cos for |x| <= pi/4, without a branch, so that the points of a lane overlap.
-// With z = x^2: sin x = x + x z S(z), cos x = (1 - z/2) + (z^2 C(z) + the rounding error
-// of 1 - z/2).  S (degree 6) and C (degree 5) interpolate the exact series at the Chebyshev
-// nodes of [0, (pi/4)^2]; truncation below 1e-18, results within 0.55 ulp like the library's.
-__device__ __forceinline__ void sincos_small(double x, double* s, double* c) {
-  const double z = x * x;
-  double p = -7.586691094197958e-13;
-  p = fma(p, z, 1.6058531516797758e-10);
-  p = fma(p, z, -2.5052106231802837e-08);
-  p = fma(p, z, 2.7557319219337312e-06);
-  p = fma(p, z, -0.00019841269841265063);
-  p = fma(p, z, 0.008333333333333331);
-  p = fma(p, z, -0.16666666666666666);
-  *s = fma(x * z, p, x);
-  double q = -1.1382623647474604e-11;
-  q = fma(q, z, 2.087614614655861e-09);
-  q = fma(q, z, -2.7557317271145144e-07);
-  q = fma(q, z, 2.480158729876456e-05);
-  q = fma(q, z, -0.0013888888888887398);
-  q = fma(q, z, 0.041666666666666664);
-  const double h = fma(-0.5, z, 1.0);
-  *c = h + fma(z * z, q, fma(-0.5, z, 1.0 - h));
 }
 
 // v *= exp(q |v|^2): a step of the self-phase modulated pump.  q is purely imaginary for a
