@@ -42,9 +42,9 @@ struct MultiLaunch {
   static constexpr int THREADS = FORM == MULTI_MODES ? P::THREADS : T;
   static constexpr int WAVES = FORM == MULTI_MODES ? (P::LEAN ? 4 : 2) : FORM == MULTI_TAB && L == 12 ? 2 : 0;
   static constexpr int LDS = FORM == MULTI_MODES ? (int)(P::LDS_BYTES / sizeof(cplx)) : FftShape<L>::lds_elems;
-  static constexpr int TW = FORM == MULTI_MODES ? 1
-                            : FORM == MULTI_TAB ? TabPolicy<L, false>::TW_ELEMS
-                                                : PropTw<L>::LDS_ELEMS;
+  static constexpr bool TW_LDS = FORM == MULTI_TAB ? TabPolicy<L, false>::TW_LDS
+                                                   : FORM != MULTI_MODES && !std::is_same<M, MChi3GNLSE>::value;
+  static constexpr int TW = TW_LDS ? PropTw<L>::LDS_ELEMS : 1;
 };
 
 // Workgroups take instances from the class's queue (one atomic counter) until it is
@@ -58,7 +58,7 @@ __global__ void __launch_bounds__((MultiLaunch<M, L, FORM>::THREADS), (MultiLaun
   __shared__ cplx twl[ML::TW];
   __shared__ int item;
   const int t = threadIdx.x;
-  if constexpr (FORM < MULTI_MODES || (FORM == MULTI_TAB && TabPolicy<L, false>::TW_LDS)) fill_twiddle_lds<L>(twl, tw);
+  if constexpr (ML::TW_LDS) fill_twiddle_lds<L>(twl, tw);
   for (;;) {
     __syncthreads();  // the previous instance's readers of `item` are done
     if (t == 0) item = atomicAdd(counter, 1);
@@ -103,7 +103,7 @@ __global__ void __launch_bounds__((MultiLaunch<M, L, FORM>::THREADS), (MultiLaun
     } else if constexpr (FORM == MULTI_TAB) {
       tab_field<L, false>(kp, 0, true, t, lds, twl);
     } else if constexpr (std::is_same<M, MChi3GNLSE>::value) {
-      gnlse_field<L>(kp, 0, true, t, lds, twl);
+      gnlse_field<L>(kp, 0, true, t, lds);
     } else {
       prop_field<M, L, FORM == MULTI_INLINE>(kp, 0, true, t, lds, twl);
     }

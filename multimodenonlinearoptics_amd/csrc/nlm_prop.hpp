@@ -486,8 +486,7 @@ __device__ __forceinline__ void gnlse_stage(const cplx (&y)[8], double r, cplx (
 // steps: 5.70 -> 3.43.  Up to N = 2048 rows and addresses stay in registers, AGPRs included
 // (fetched and formed per stage: 5.66 ms).
 template <int L>
-__device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool active, int t0, cplx* buf,
-                                            const cplx* twl) {
+__device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool active, int t0, cplx* buf) {
   using F = FftShape<L>;
   constexpr int N = F::N;
   int t = t0;
@@ -495,7 +494,7 @@ __device__ __forceinline__ void gnlse_field(const KParams& kp, int field, bool a
   // N = 4096: with the rows fetched and addresses formed per stage the twiddles fit registers
   // (with rows and addresses held and twiddles in LDS 92 us per step of 64 rows, so 70)
   typename std::conditional<FftShape<L>::LOG == 12, RegTwiddles<L>, typename PropTw<L>::type>::type tw;
-  init_twiddles<L>(tw, kp.tw, twl, t);
+  init_twiddles<L>(tw, kp.tw, nullptr, t);  // no size keeps them in LDS
   SpectralRow<L, PropTw<L>::LEAN> ds, ram, flt;
   ds.init(kp.dstep, t);
   ram.init(kp.raman, t);
@@ -560,11 +559,9 @@ __global__ void __launch_bounds__(Launch<L>::THREADS) k_prop_gnlse(KParams kp) {
   using F = FftShape<L>;
   constexpr int T = F::T, FPB = Launch<L>::FPB;
   __shared__ cplx lds[FPB * F::lds_elems];
-  __shared__ cplx twl[PropTw<L>::LDS_ELEMS];
-  fill_twiddle_lds<L>(twl, kp.tw);
   const int lf = threadIdx.x / T, t = threadIdx.x % T;
   const int field = blockIdx.x * FPB + lf;
-  gnlse_field<L>(kp, field, field < kp.nFields, t, lds + lf * F::lds_elems, twl);
+  gnlse_field<L>(kp, field, field < kp.nFields, t, lds + lf * F::lds_elems);
 }
 
 typedef void (*prop_fn)(const KParams&, int grid, hipStream_t);
