@@ -465,9 +465,7 @@ struct AnyLaunch {
 
 int any_launch(nlm_plan_s* p, DevBuf<cplx>* own, int NS, int N, long items, AnyLaunch* out, bool may_alloc = true) {
   const size_t bytes = (size_t)2 * NS * N * sizeof(cplx);
-  int cus = 256, dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  if (cus <= 0) cus = 256;
+  const int cus = device_cus();
   if (bytes <= ANY_LDS_BYTES) {
     const long per = std::max<long>(1, (long)(160 * 1024 / bytes));
     out->grid = (int)std::max<long>(1, std::min<long>(items, cus * std::min<long>(per, 8)));

@@ -710,8 +710,7 @@ bool nlm_big_supported(int model, int L) { return model == NLM_CHI3GNLSE && (L =
 // under a caller's stream capture, where it is one plain launch.  At N = 4096 it is the faster
 // one (4 rows 55 against 61, 64 rows 70 against 95).
 bool nlm_big_better(nlm_plan* p, int rows) {
-  constexpr int CUS = 256;
-  if (p->model != NLM_CHI3GNLSE || p->L != 13 || p->nZ < 2 || rows > CUS) return false;
+  if (p->model != NLM_CHI3GNLSE || p->L != 13 || p->nZ < 2 || rows > device_cus()) return false;
   if (stream_capturing(p->stream)) return false;
   if (ensure_state(p, rows) == NLM_OK) return true;
   (void)hipGetLastError();

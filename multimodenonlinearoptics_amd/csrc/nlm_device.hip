@@ -851,7 +851,7 @@ int launch_prop_kernel_tab(nlm_plan* p, const KParams& kp0, cplx* tab, bool may_
     fn = nlm_pick_prop_tab(p->L);
     // few fields: four points per lane as long as that is at most two waves per CU (N = 128, 2000
     // fields, 500 of the eight-point waves: 1.28 against 1.42 ms)
-    if (p->L <= 8 && grid <= 256) fn = nlm_pick_prop_quad(p->L);
+    if (p->L <= 8 && grid <= device_cus()) fn = nlm_pick_prop_quad(p->L);
     const int forced = env_int("NLM_FFT_SCHEDULE", -1);
     if (forced >= 0) {
       if (prop_fn f = nlm_pick_prop_tab_variant(p->L, forced)) fn = f;
@@ -967,6 +967,12 @@ extern "C" int nlm_grid_download(nlm_plan* p, int mode, double* sf, double* st) 
   const size_t cnt = (size_t)p->nZ * p->N, off = (size_t)mode * cnt;
   const HostCopy out[2] = {{sf, p->gridF.p + off, cnt * sizeof(cplx)}, {st, p->gridT.p + off, cnt * sizeof(cplx)}};
   return nlm_to_host(out, 2, p->stream);
+}
+
+int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  return cus > 0 ? cus : 256;
 }
 
 bool stream_capturing(hipStream_t s) {

@@ -74,11 +74,12 @@ inline bool mix_split(int q, int maxParts, int* parts, int* n) {
 // estimated time is taken: a wave's points per stage (FP64 and LDS work) plus a
 // latency per exchange (larger where its barrier joins several waves; fitted to
 // the times above), times the rounds of waves that the fields make on the
-// chip's 1024 SIMDs.  Few fields thus get more lanes and fewer points per lane, many
+// device's SIMDs (1024).  Few fields thus get more lanes and fewer points per lane, many
 // fields the larger radices.
 inline bool mix_plan(int N, int groups, long fields, bool gnlse, MixPlan* out) {
   static const int first[] = {10, 9, 8, 6, 5, 4, 3, 2};
   if (N < 8) return false;
+  const double simds = 4.0 * device_cus();
   double best = 0;
   MixPlan p;
   for (int R : first) {
@@ -114,7 +115,7 @@ inline bool mix_plan(int N, int groups, long fields, bool gnlse, MixPlan* out) {
     }
     cost += (p.waveFft ? 400.0 : 900.0) * (p.nMid + 1);
     const double waves = (double)((fields + p.FPB - 1) / p.FPB) * (p.threads / 64);
-    cost *= std::max(1.0, waves / 1024.0);
+    cost *= std::max(1.0, waves / simds);
     if (best == 0 || cost < best) {
       best = cost;
       *out = p;

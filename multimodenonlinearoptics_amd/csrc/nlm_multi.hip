@@ -98,12 +98,6 @@ struct nlm_multi_s {
 static std::mutex g_tune_mu;
 static std::map<std::tuple<int, int, int, int>, int> g_tuned;  // (model, L, form, count) -> grid
 
-static int device_cus() {
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-  return cus > 0 ? cus : 256;
-}
-
 static void launch_stage(nlm_multi_s* m, const MultiClass& c, const cplx* tw, hipStream_t s) {
   nlm_multi_stage(c.stage, c.model, c.L, m->inst.p, m->chunks.p + 2 * (size_t)c.chunkOff, c.nChunks, tw, s);
 }

@@ -580,6 +580,9 @@ prop_fn nlm_pick_prop(int model, int L);
 // Step-propagator kernel (one signal mode) for log2 N = L, and its table builder.
 prop_fn nlm_pick_prop_tab(int L);
 prop_fn nlm_pick_prop_quad(int L);
+// CUs of the current device, by which the forms of a launch are chosen (256 where it is not
+// partitioned)
+int device_cus();
 // schedule variant 0..3 of the table kernel (see FftShape); nullptr where a
 // variant does not exist or equals the default
 prop_fn nlm_pick_prop_tab_variant(int L, int variant);
