@@ -57,19 +57,16 @@ static void launch_tab(const KParams& kp, int grid, hipStream_t s) {
 }
 
 // The form of a launch (TabPolicy): the two-waves form where it exists and the
-// launch's waves exceed one per SIMD.  N = 1024 with at most one field per CU is
-// scheduled for one wave per SIMD (one field 0.490 -> 0.472 ms of 199 steps, 200
-// fields 0.510 -> 0.493; no gain with 512 fields).  N = 2048 gains nothing by it (one field
-// 0.718 -> 0.718, 8 fields 0.731 -> 0.735, 256 fields 0.774 -> 0.783).
+// launch's waves exceed one per SIMD.  Asking for one wave per SIMD where a launch of
+// few fields leaves the chip idle changes nothing (199 steps of 1, 8, 64, 200 fields, ms:
+// N = 1024 0.479 / 0.484 / 0.487 / 0.499 with it, 0.479 / 0.484 / 0.487 / 0.498 without;
+// N = 2048 0.718 / 0.735 / 0.729 / 0.737 and 0.718 / 0.731 / 0.729 / 0.737).
 template <int L>
 static void launch_prop_tab(const KParams& kp, int grid, hipStream_t s) {
-  constexpr int LOG = FftShape<L>::LOG;
   if constexpr (TabPolicy<L, false>::HOOK) {
     launch_tab<L, false, 2>(kp, grid, s);
   } else if constexpr (TabPolicy<L, true>::HOOK) {
-    const int cus = device_cus();
-    if ((long)grid * (Launch<L>::THREADS / 64) > 4 * cus) launch_tab<L, true, 2>(kp, grid, s);
-    else if (LOG == 10 && grid <= cus) launch_tab<L, false, LOG == 10 ? 1 : 0>(kp, grid, s);
+    if ((long)grid * (Launch<L>::THREADS / 64) > 4 * device_cus()) launch_tab<L, true, 2>(kp, grid, s);
     else launch_tab<L, false, 0>(kp, grid, s);
   } else {
     launch_tab<L, false, 0>(kp, grid, s);
