@@ -2,6 +2,8 @@
 would need, which stageLimit sets: pump rows generated in the kernel ("inline"), one-mode media
 fed from their pump grids ("field"), and a limit that holds only the largest class.  Every
 instance against the oracle at the engine's rel. L2 of 1e-10."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -90,3 +92,43 @@ def test_staging_that_cannot_be_had(nlm):
         got.append([b.output(i) for i in (0, count - 1, count)])
     for a, c in zip(*got):
         assert np.isfinite(a).all() and np.array_equal(a, c)
+
+
+class Item(C.Structure):
+    _fields_ = [("plan", C.c_void_p), ("input", C.c_void_p), ("cols", C.c_int32), ("in_time", C.c_int32),
+                ("input_mode", C.c_int32), ("n_out", C.c_int32), ("outputs", C.c_int32 * 4), ("envelope", C.c_void_p),
+                ("disp_pump", C.c_void_p), ("dzp", C.c_double), ("strength", C.c_void_p)]
+
+
+@pytest.mark.parametrize("limit,form", [(-1, 3), (0, 0)])
+def test_pump_grids_of_pdc_media(nlm, limit, form):
+    """Chi2PDC media without an envelope, through the C interface: step tables made of their pump
+    grids, or the grids read in the kernel; lengths of 1 step, one chunk and a partial one."""
+    from multimodenonlinearoptics_amd import capi
+    L = capi.lib()
+    L.nlm_multi_create_staged.argtypes = [C.c_int, C.c_void_p, C.c_int, C.c_int64, C.c_void_p]
+    L.nlm_multi_output.argtypes = [C.c_void_p, C.c_int, C.c_void_p]
+    media, xs, items = [], [], []
+    for j, (N, nZ) in enumerate([(32, 2), (64, 17), (64, 40), (1024, 19), (4096, 5)]):
+        m = nlm.Chi2PDC(**small_case("Chi2PDC", nlm, N=N, nZ=nZ, seed=j, poled=False)[1])
+        m.runPumpSimulation()
+        media.append(m)
+        xs.append(random_inputs("Chi2PDC", N, 1, seed=j)[0])
+        it = Item(m.planHandle(), xs[-1].ctypes.data, N, 1, 0, 1)
+        items.append(it)
+        capi.check(L.nlm_plan_sync(C.c_void_p(m.planHandle())))
+    arr, b = (Item * len(items))(*items), C.c_void_p()
+    capi.check(L.nlm_multi_create_staged(len(items), arr, 0, limit, C.byref(b)))
+    try:
+        for c in range(L.nlm_multi_classes(b)):
+            f = C.c_int32()
+            capi.check(L.nlm_multi_form(b, c, C.byref(f), None))
+            assert f.value == form
+        capi.check(L.nlm_multi_launch(b))
+        capi.check(L.nlm_multi_sync(b, None))
+        for i, (m, x) in enumerate(zip(media, xs)):
+            out = np.empty(x.size, np.complex128)
+            capi.check(L.nlm_multi_output(b, i, out.ctypes.data))
+            assert rel_l2(out, m.batchSignalSimulation(x[None, :], inTimeDomain=True)[0]) < 1e-12, i
+    finally:
+        L.nlm_multi_destroy(b)
