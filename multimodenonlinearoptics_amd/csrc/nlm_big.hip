@@ -717,7 +717,7 @@ bool nlm_big_better(nlm_plan* p, int rows) {
   return false;
 }
 
-// Batch propagation of a Chi3GNLSE plan with nFreqs 16384 or 32768 (see above).
+// Batch propagation of a Chi3GNLSE plan with nFreqs 8192 (nlm_big_better), 16384 or 32768.
 // in / out are device arrays with the layout of nlm_batch_dev.
 int nlm_big_batch(nlm_plan* p, const cplx* in, int rows, int cols, int inTime, int inPos, int nOut, int outPos,
                   cplx* out) {

@@ -75,7 +75,7 @@ struct nlm_plan_s {
   DevBuf<cplx> ckpt, gG, gC, gS, gcoefPart, gcoef, gpumpPart, gpump, gF0Part, gF0, gtmp, gslice;
   DevBuf<cplx> scale;
   DevBuf<cplx> cascade[2][2];  // products of nlm_greens_cascade whose last plan this is
-  // staged transform for Chi3GNLSE with nFreqs > 8192 (nlm_big.hip)
+  // staged transform for Chi3GNLSE batches with nFreqs >= 8192 and the gradient (nlm_big.hip)
   DevBuf<cplx> bigState, bigH;
   int ramanReal = 0;  // the Raman response is the spectrum of a real one
   DevBuf<BigArgs> bigArgs;
@@ -117,9 +117,10 @@ int scratch_mark(nlm_plan_s* p);
 int get_twiddles(int n, const cplx** out);
 // input channel feeding each mode (-1: none), src/_NonlinearMedium.hpp:164-198
 void input_channels(int nS, int nCh, int inputMode, int* inPos);
-// Chi3GNLSE batches with nFreqs 16384 / 32768 (nlm_big.hip)
+// Chi3GNLSE batches staged through memory (nlm_big.hip): nFreqs 16384 / 32768, which no
+// workgroup can hold
 bool nlm_big_supported(int model, int L);
-// 8192, whose batches run staged too although one workgroup could hold a field
+// and 8192 up to a row per CU, although one workgroup could hold a field
 bool nlm_big_better(nlm_plan_s* p, int rows);
 int nlm_big_batch(nlm_plan_s* p, const cplx* in, int rows, int cols, int inTime, int inPos, int nOut, int outPos,
                   cplx* out);
