@@ -14,11 +14,12 @@
 //
 // Every signal mode of a medium has lanes of its own (nlm_modes.hpp).
 //
-// What bounds it: like every kernel of this engine, a wave's FP64 instructions (4
-// cycles each) plus its 16-byte LDS accesses (~30 cycles each when nothing else runs
-// on the SIMD).  nlm_any.hip's general kernel, which this replaces for these
-// lengths, forms one output element per lane and pass: R table twiddles, R LDS reads
-// and R complex products for every element instead of one butterfly per R elements.
+// What bounds it: a wave's FP64 instructions (4 cycles each) and its 16-byte LDS accesses
+// (~30 cycles each when nothing else runs on the SIMD), 70 % of its cycles at N = 600 by the
+// counters, and the table reads, index arithmetic and stores between them.  nlm_any.hip's
+// general kernel, which this replaces for these lengths, forms one output element per lane
+// and pass: R table twiddles, R LDS reads and R complex products for every element instead
+// of one butterfly per R elements.
 // Measured, kernel ms before -> now: Chi2PDC Green's function N = 600, nZ = 200
 // (1200 fields, 10 x 6 x 10, one wave each) 9.16 -> 1.41; in the same launch R = 5
 // takes 2.41 and R = 2 3.69, while one field alone takes 1.15 (R = 5), 1.13 (R = 2)
