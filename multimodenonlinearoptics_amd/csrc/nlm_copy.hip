@@ -215,6 +215,15 @@ hipError_t large(Staging* st, char* host, const char* dev, size_t bytes, hipStre
   return hipSuccess;
 }
 
+// Whether the runtime knows the memory (pinned, managed, a device's): its own copy then goes
+// there directly.  Two results of 67 MB into pinned arrays 4.32 -> 2.37 ms.
+bool known(const void* host) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, host) == hipSuccess) return a.type != hipMemoryTypeUnregistered;
+  (void)hipGetLastError();
+  return false;
+}
+
 // Without a staging area (no pinned memory left): the runtime's own copies.
 hipError_t plain(const HostCopy* items, int n, hipStream_t s) {
   hipError_t e = hipSuccess;
@@ -246,7 +255,7 @@ int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     size_t o = 0;
     for (int i = first; i < end && e == hipSuccess; i++) {
-      if (!items[i].host || items[i].bytes > SMALL) continue;
+      if (!items[i].host || items[i].bytes == 0 || items[i].bytes > SMALL || known(items[i].host)) continue;
       memcpy(items[i].host, st->buf + o, items[i].bytes);
       o += items[i].bytes;
     }
@@ -256,7 +265,9 @@ int nlm_to_host(const HostCopy* items, int n, hipStream_t s) {
   for (int i = 0; i < n && e == hipSuccess; i++) {
     const HostCopy& c = items[i];
     if (!c.host || c.bytes == 0) continue;
-    if (c.bytes >= LARGE) {
+    if (known(c.host)) {
+      e = hipMemcpyAsync(c.host, c.dev, c.bytes, hipMemcpyDeviceToHost, s);
+    } else if (c.bytes >= LARGE) {
       flush(i);
       first = i + 1;
       if (e == hipSuccess) e = large(st, (char*)c.host, (const char*)c.dev, c.bytes, s);

@@ -82,6 +82,19 @@ int main(int argc, char** argv) {
       copy({100, 5 * MB}, &s, r);
     }
     CHECK(fake::areas == 2);
+  } else if (what == "pinned") {
+    // two results in pinned memory, one large and one small, between two in ordinary memory
+    std::vector<char> dev(5 * MB, 7), pin(6 * MB, 0), a(100, 0), b(4 * MB, 0);
+    fake::pinned = pin.data();
+    fake::pinnedEnd = pin.data() + pin.size();
+    const HostCopy c[] = {{a.data(), dev.data(), 100}, {pin.data(), dev.data(), 5 * MB},
+                          {b.data(), dev.data(), 4 * MB}, {pin.data() + 5 * MB, dev.data(), 200}};
+    CHECK(nlm_to_host(c, 4, &s) == NLM_OK);
+    CHECK(fake::pinnedCopies == 2);
+    for (size_t i = 0; i < pin.size(); i++)
+      if (pin[i] != (i < 5 * MB + 200 ? 7 : 0)) failures++;
+    for (char x : a) failures += x != 7;
+    for (char x : b) failures += x != 7;
   } else {
     std::printf("unknown scenario\n");
     return 2;

@@ -7,6 +7,10 @@
 #include <cstring>
 
 enum hipError_t { hipSuccess = 0, hipErrorInvalidValue = 1, hipErrorOutOfMemory = 2, hipErrorInvalidHandle = 400 };
+enum hipMemoryType { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1, hipMemoryTypeDevice = 2 };
+struct hipPointerAttribute_t {
+  hipMemoryType type;
+};
 enum hipMemcpyKind { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
 constexpr unsigned hipHostMallocDefault = 0, hipEventDisableTiming = 2;
 
@@ -24,6 +28,10 @@ inline thread_local int device = 0;
 inline thread_local hipError_t last = hipSuccess;
 inline std::atomic<bool> failHostMalloc{false}, failEventCreate{false};
 inline std::atomic<int> areas{0}, events{0};
+// a caller's pinned memory, and the copies that went there
+inline const char *pinned = nullptr, *pinnedEnd = nullptr;
+inline std::atomic<int> pinnedCopies{0};
+inline bool isPinned(const void* p) { return p >= pinned && p < pinnedEnd; }
 inline hipError_t ret(hipError_t e) {
   if (e != hipSuccess) last = e;
   return e;
@@ -75,7 +83,12 @@ inline hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 }
 inline hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
+  a->type = fake::isPinned(p) ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+  return hipSuccess;
+}
 inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
+  if (fake::isPinned(dst)) fake::pinnedCopies++;
   std::memcpy(dst, src, n);
   return hipSuccess;
 }

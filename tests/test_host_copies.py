@@ -44,3 +44,8 @@ def test_no_pinned_memory(driver):
 def test_stream_of_another_device(driver):
     """A plan's results while another device is the current one, which stays so."""
     run(driver, "device")
+
+
+def test_results_in_pinned_memory(driver):
+    """A caller's pinned memory is filled by one copy of the runtime's each, not by way of the area."""
+    run(driver, "pinned")
