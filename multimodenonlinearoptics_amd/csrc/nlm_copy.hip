@@ -6,15 +6,18 @@
 // pinned staging area in 1 MB pieces, two per participant in flight, and the caller and up to
 // three helper threads move the pieces to the destination.  That pays from about 3 MB (a
 // batch's result of 6.2 MB 816 -> 766 us for the call, 12.5 MB 2.24 -> 1.35 ms, two of 16 MB 2.02 ->
-// 1.28; at 2 MB 50 us slower).  Small results are gathered in the area and share one wait;
-// between the two the runtime's own copy is used, as for every upload, whose source pages are
-// there already (in pieces by the helpers a 6.2 MB input made the call 766 -> 1395 us).
+// 1.28; at 2 MB 50 us slower), and for one caller at a time: callers that come meanwhile take the
+// runtime's copy, since several at once are bound by the transfers (four threads with two
+// results of 16.8 MB each: 3.23 ms a round, 3.22 all by the runtime, 3.93 by way of the area).
+// Small results are gathered in the area and share one wait; between the two the runtime's own
+// copy is used, as for every upload, whose source pages are there already (in pieces by the helpers a 6.2 MB input made the call 766 -> 1395 us).
 // Calls, ms before -> now: Chi2PDC Green's N = 512 (C, S of 4 MB each) 2.63 -> 2.37, N =
 // 32 0.116 -> 0.080; Chi3 z-grids N = 512, nZ = 1000 (48 MB) 11.4 -> 10.6.
 #include <sys/types.h>
 #include <unistd.h>
 
 #include <algorithm>
+#include <atomic>
 #include <condition_variable>
 #include <cstring>
 #include <mutex>
@@ -188,6 +191,8 @@ hipError_t share(Staging* st, char* host, const char* dev, size_t bytes, int par
   return e;
 }
 
+std::atomic<int> g_large{0};  // large copies under way in the process
+
 hipError_t large(Staging* st, char* host, const char* dev, size_t bytes, hipStream_t s) {
   struct Shares : Job {
     Staging* st;
@@ -209,7 +214,11 @@ hipError_t large(Staging* st, char* host, const char* dev, size_t bytes, hipStre
   job.dev = dev;
   job.bytes = bytes;
   job.s = s;
-  if (!helpers().run(job)) return share(st, host, dev, bytes, 0, 1, s);
+  struct Entered {
+    const int others = g_large.fetch_add(1);
+    ~Entered() { g_large.fetch_sub(1); }
+  } entered;
+  if (entered.others > 0 || !helpers().run(job)) return hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s);
   for (hipError_t e : job.errs)
     if (e != hipSuccess) return e;
   return hipSuccess;

@@ -46,6 +46,18 @@ static void copy(const std::vector<size_t>& sizes, FakeStream* s, unsigned seed)
 
 constexpr size_t MB = (size_t)1 << 20;
 
+// A second caller's large copy, in the middle of a first one's
+static void second() {
+  std::thread([] {
+    FakeStream s{0};
+    std::vector<char> dev(4 * MB, 3), host(4 * MB, 0);
+    fake::watched = host.data();
+    const HostCopy c = {host.data(), dev.data(), host.size()};
+    CHECK(nlm_to_host(&c, 1, &s) == NLM_OK);
+    CHECK(fake::watchedCopies == 1 && dev == host);
+  }).join();
+}
+
 int main(int argc, char** argv) {
   const std::string what = argc > 1 ? argv[1] : "";
   FakeStream s{0};
@@ -95,6 +107,13 @@ int main(int argc, char** argv) {
       if (pin[i] != (i < 5 * MB + 200 ? 7 : 0)) failures++;
     for (char x : a) failures += x != 7;
     for (char x : b) failures += x != 7;
+  } else if (what == "two callers") {
+    for (int r = 1; r <= 3; r++) {
+      fake::watchedCopies = 0;
+      fake::onCopy = second;
+      copy({9 * MB}, &s, r);
+    }
+    CHECK(threadsMade == 3 + 3);  // helpers, and the second callers themselves
   } else {
     std::printf("unknown scenario\n");
     return 2;

@@ -31,6 +31,10 @@ inline std::atomic<int> areas{0}, events{0};
 // a caller's pinned memory, and the copies that went there
 inline const char *pinned = nullptr, *pinnedEnd = nullptr;
 inline std::atomic<int> pinnedCopies{0};
+// copies whose destination is `watched`; a call made from the next copy, once
+inline const void* watched = nullptr;
+inline std::atomic<int> watchedCopies{0};
+inline std::atomic<void (*)()> onCopy{nullptr};
 inline bool isPinned(const void* p) { return p >= pinned && p < pinnedEnd; }
 inline hipError_t ret(hipError_t e) {
   if (e != hipSuccess) last = e;
@@ -89,6 +93,8 @@ inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* 
 }
 inline hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {
   if (fake::isPinned(dst)) fake::pinnedCopies++;
+  if (dst == fake::watched) fake::watchedCopies++;
+  if (void (*f)() = fake::onCopy.exchange(nullptr)) f();
   std::memcpy(dst, src, n);
   return hipSuccess;
 }

@@ -49,3 +49,8 @@ def test_stream_of_another_device(driver):
 def test_results_in_pinned_memory(driver):
     """A caller's pinned memory is filled by one copy of the runtime's each, not by way of the area."""
     run(driver, "pinned")
+
+
+def test_second_caller_takes_the_plain_copy(driver):
+    """While one caller's copy goes by way of the area, another's is the runtime's."""
+    run(driver, "two callers")
