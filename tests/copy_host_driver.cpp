@@ -114,6 +114,15 @@ int main(int argc, char** argv) {
       copy({9 * MB}, &s, r);
     }
     CHECK(threadsMade == 3 + 3);  // helpers, and the second callers themselves
+  } else if (what == "one cpu") {
+    cpu_set_t all, one;
+    sched_getaffinity(0, sizeof all, &all);
+    CPU_ZERO(&one);
+    for (int k = 0; k < CPU_SETSIZE && CPU_COUNT(&one) == 0; k++)
+      if (CPU_ISSET(k, &all)) CPU_SET(k, &one);
+    sched_setaffinity(0, sizeof one, &one);
+    second();
+    CHECK(threadsMade == 1);  // the caller itself
   } else {
     std::printf("unknown scenario\n");
     return 2;

@@ -8,7 +8,8 @@ import subprocess
 import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+pytestmark = [pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available"),
+              pytest.mark.skipif(len(os.sched_getaffinity(0)) < 3, reason="helpers need three CPUs")]
 
 
 @pytest.fixture(scope="module")
@@ -54,3 +55,8 @@ def test_results_in_pinned_memory(driver):
 def test_second_caller_takes_the_plain_copy(driver):
     """While one caller's copy goes by way of the area, another's is the runtime's."""
     run(driver, "two callers")
+
+
+def test_one_cpu(driver):
+    """A process on one CPU starts no helpers, its copies are the runtime's."""
+    run(driver, "one cpu")
