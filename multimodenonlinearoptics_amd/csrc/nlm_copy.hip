@@ -8,7 +8,7 @@
 // batch's result of 6.2 MB 816 -> 766 us for the call, 12.5 MB 2.24 -> 1.35 ms, two of 16 MB 2.02 ->
 // 1.28; at 2 MB 50 us slower), and for one caller at a time: callers that come meanwhile take the
 // runtime's copy, since several at once are bound by the transfers (four threads with two
-// results of 16.8 MB each: 3.23 ms a round, 3.22 all by the runtime, 3.93 by way of the area).
+// results of 16.8 MB each: 3.23 ms a pass, 3.22 all by the runtime, 3.93 by way of the area).
 // Small results are gathered in the area and share one wait; between the two the runtime's own
 // copy is used, as for every upload, whose source pages are there already (in pieces by the helpers a 6.2 MB input made the call 766 -> 1395 us).
 // Calls, ms before -> now: Chi2PDC Green's N = 512 (C, S of 4 MB each) 2.63 -> 2.37, N =
