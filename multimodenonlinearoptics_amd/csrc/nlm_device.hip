@@ -492,6 +492,8 @@ extern "C" int nlm_plan_create(const nlm_plan_desc* d, nlm_plan** out) {
   p->stream = p->own;
   for (auto& ev : p->ev)
     if (hipEventCreate(&ev) != hipSuccess) return fail(set_err(NLM_DEVICE_ERROR, "hipEventCreate failed"));
+  if (hipEventCreateWithFlags(&p->scratchDone, hipEventDisableTiming) != hipSuccess)
+    return fail(set_err(NLM_DEVICE_ERROR, "hipEventCreate failed"));
   if ((e = get_twiddles(p->N, &p->tw))) return fail(e);
   const size_t nsN = (size_t)p->nS * p->N;
   if ((e = upload(p->dstep, d->disp_step, nsN, p->stream))) return fail(e);
@@ -990,7 +992,6 @@ int scratch_wait(nlm_plan* p) {
 int scratch_mark(nlm_plan* p) {
   if (!p->scratchUsed) return NLM_OK;
   p->scratchUsed = false;
-  if (!p->scratchDone) HIP_TRY(hipEventCreateWithFlags(&p->scratchDone, hipEventDisableTiming));
   HIP_TRY(hipEventRecord(p->scratchDone, p->stream));
   p->scratchBusy = true;
   return NLM_OK;
